@@ -228,10 +228,10 @@ typedef struct rmd_options {
   int32_t search_mode;           /* list search: 1 one wave per atom, 2 one wave
                                     per cell, 3 by the plan's cell occupancy,
                                     0 = tuned                                  */
-  int32_t pme_bins;              /* PME planes of a single system: 1 bin the
-                                    atoms by x plane, 2 every plane scans every
-                                    atom, 3 by atom count, 0 = tuned (batch
-                                    members always bin)                        */
+  int32_t pme_bins;              /* PME planes of a single system: 1 each
+                                    finds its atoms by the cell list, 2 it
+                                    scans every atom, 3 by atom count, 0 =
+                                    tuned (batch members bin by x plane)       */
 } rmd_options;
 void rmd_options_default(rmd_options *options);
 
@@ -337,7 +337,7 @@ typedef struct rmd_diagnostics {
   double pme_alpha;
   int32_t lanes_per_atom;
   int32_t water_units, cluster_units, free_units;
-  int32_t pme_planes; /* 1: plane PME pipeline, 0: line pipeline */
+  int32_t pme_planes; /* 1: plane PME pipeline, 0: slab pipeline */
   int32_t cell_reach;      /* the cell plan's stencil reach (1: the reference's plan) */
   int32_t search_by_cell;  /* 1: the list search runs one wave per cell */
   int64_t steps_since_barostat; /* steps run since the last volume move (a
@@ -416,8 +416,8 @@ int rmd_set_graphs(rmd_ctx *ctx, int32_t enabled);
 int rmd_set_concurrent_forces(rmd_ctx *ctx, int32_t enabled);
 /* PME pipeline: 0 automatic (planes when one x plane of the grid fits in
  * LDS; mode 4 for a single system of at most 32 x planes that does not bin),
- * 1 planes (RMD_E_INVALID when it does not fit), 2 lines, 3 planes with
- * every plane scanning every atom (no atom bins, which large single systems
+ * 1 planes (RMD_E_INVALID when it does not fit), 2 slabs (passes of line tiles), 3 planes with
+ * every plane scanning every atom (not by cells, which large single systems
  * and batch members build by default), 4 as 3 with force-only evaluations
  * folding the x lines into the plane gathers (one launch fewer per
  * evaluation; RMD_E_INVALID beyond 32 x planes or for a batch member).

@@ -11,7 +11,7 @@ workloads under candidate shapes and keeps the fastest:
 - skin: the Verlet skin, which trades list rebuilds against list length
   (the list is rebuilt on a device-side displacement test, so the skin is a
   speed choice, not a correctness one);
-- pme_bins: whether a single system's PME planes read per-plane atom bins or
+- pme_bins: whether a single system's PME planes find their atoms by cells or
   scan every atom.
 
 Workload classes: single systems of 1,189, 2,854, 12,472 and 100,200 atoms
@@ -219,7 +219,7 @@ def header(rows):
         "// batches (kind 1). lanes: direct-space lanes per atom; reach: the widest cell",
         "// stencil reach the plan may take; searchMode: 0 by cell occupancy, 1 one wave",
         "// per atom, 2 one wave per cell; skin: nm when the caller asks for the tuned",
-        "// skin (0: the reference's skinFor); pmeBins: 0 by atom count, 1 atom bins,",
+        "// skin (0: the reference's skinFor); pmeBins: 0 by atom count, 1 by cells,",
         "// 2 every plane scans every atom.",
         "struct TunedShape {",
         "  int kind, minAtoms, lanes, reach, searchMode;",

@@ -194,7 +194,7 @@ struct rmd_ctx {
   int windowAttempts = 0, windowAccepted = 0;
   double volumeScale = -1;
   int64_t stepsSinceBarostat = 0;
-  int pmeBinned = 0;   // whether the plane pipeline bins its atoms (set at creation)
+  int pmeAtoms = 0;    // how the plane pipeline finds its atoms, PME_ATOMS_* (set at creation)
   int pmeFolded = 0;   // whether force-only evaluations fold the x lines into the gathers (set at creation)
   int reachMax = 0;    // the cell plan's widest reach (0: CELL_REACH_MAX)
   int searchMode = 0;  // 0 by occupancy, 1 per atom, 2 per cell where the launch covers the cells
@@ -534,11 +534,10 @@ __global__ void setStepKernel(Scalars *sc, long long step) { sc->step = step; }
 // and PME forward planes as one launch after the list rebuild, then the rest
 // of PME, all on the context's stream: a captured step runs forked branches
 // one after another, so separate launches cost the sum of their durations,
-// where one launch overlaps them. Otherwise PME, the longest branch, stays on
-// the context's stream, and the neighbour-list branch (rebuild + direct
-// space) and the bonded terms, which read only the positions, run on side
-// streams forked after the integrator and joined before anything that reads
-// the forces. Forces are int64 atomics and every energy has its own slot row,
+// where one launch overlaps them. Otherwise the cell list comes first; PME,
+// the longest branch, stays on the context's stream, and the list search with
+// the direct space, and the bonded terms, run on side streams forked after it
+// and joined before anything that reads the forces. Forces are int64 atomics and every energy has its own slot row,
 // so the results do not depend on the overlap.
 // `molecular`: energies with the molecular scaling term; `cellsBuilt`: the
 // step's integrator has built the cell list.
@@ -557,7 +556,8 @@ void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT],
   if (joined) {
     // the one-wave-per-atom search runs in the joined launch
     const bool searchJoined = !searchByCell(c->searchMode, d.n, c->plan.cellCount);
-    launchRebuild(d, c->stream, cellsBuilt, searchJoined);
+    if (!cellsBuilt) launchCells(d, c->stream);
+    if (!searchJoined) launchSearch(d, c->searchMode, c->stream);
     int pair = 0, bonded = 0;
     launchForcesJoined(d, c->p, (float)c->pme.alpha, rational, c->lanes, energies, c->pme.alpha, terms, c->stream,
                        &pair, &bonded, searchJoined ? 1 : 0);
@@ -568,6 +568,7 @@ void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT],
     const bool fork = c->concurrent;
     hipStream_t pmeStream = c->stream, listStream = fork ? c->side[0] : c->stream,
                 bondedStream = fork ? c->side[1] : c->stream;
+    if (!cellsBuilt) launchCells(d, c->stream);  // before the fork: PME reads the cell order too
     if (fork) {
       HIP_CHECK(hipEventRecord(c->fork, c->stream));
       HIP_CHECK(hipStreamWaitEvent(c->side[0], c->fork, 0));
@@ -583,7 +584,7 @@ void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT],
       launchBonded(d, c->pme.alpha, terms, energies, bondedStream, &b);
       setBondedSlots(b);
     }
-    launchRebuild(d, listStream, cellsBuilt);
+    launchSearch(d, c->searchMode, listStream);
     if (terms & RMD_TERM_DIRECT) {
       const int b = launchNonbonded(d, (float)c->pme.alpha, rational, c->lanes, energies, listStream);
       slots[E_LJ_DIRECT] = slots[E_COUL_DIRECT] = slots[E_DSCALE_DIRECT] = b;
@@ -1320,34 +1321,27 @@ void create(rmd_ctx *c, const System &sys, const rmd_options &o, const Streams *
   }
   const size_t grid = (size_t)p.K[0] * p.K[1] * p.K[2];
   const size_t half = (size_t)p.K[0] * p.K[1] * p.K2h;
-  p.qgrid = devAlloc<long long>(grid, c->held);
   p.rgrid = devAlloc<float>(grid, c->held);
   p.cgrid = devAlloc<float2>(half, c->held);
   p.influence = devAlloc<float>(half, c->held);
   p.piOverAlpha2 = M_PI * M_PI / (c->pme.alpha * c->pme.alpha);
   pmeConfigure(p, PME_AUTO, c->maxLds);
-  // The plane pipeline's atom bins. A small single system scans every atom
-  // per plane (one launch fewer on a short critical path); replica batches
-  // bin their members in one workgroup each, and a large single system bins
-  // its atoms in groups over the whole chip (the same results: see pme.hip).
-  p.binned = 0;
-  p.binGroups = 0;
+  // How the planes find their atoms (PME_ATOMS_*): the same results.
   if (o.pme_bins < 0 || o.pme_bins > 3)
-    throw Error(RMD_E_INVALID, "pme_bins must be 0 (tuned), 1 (bins), 2 (scan) or 3 (by atom count)");
+    throw Error(RMD_E_INVALID, "pme_bins must be 0 (tuned), 1 (cells), 2 (scan) or 3 (by atom count)");
   // bins 0 is the rule by atom count (option 3)
   const int bins = o.pme_bins == 0 ? tuned.pmeBins : o.pme_bins == 3 ? 0 : o.pme_bins;
-  const bool wide = !shared && pmeBinsFitWide(p) && (bins == 1 || (bins == 0 && d.n >= BIN_SINGLE_MIN_ATOMS));
-  if ((shared && pmeBinsFit(p, d.n)) || wide) {
-    p.binned = 1;
+  p.atoms = PME_ATOMS_SCAN;
+  if (shared && pmeBinsFit(p, d.n)) {
+    p.atoms = PME_ATOMS_BINS;
     p.binStart = devAlloc<int>(p.K[0] + 1, c->held);
     p.atomBin = devAlloc<int2>(d.nPad, c->held);
     p.binAtoms = devAlloc<int>(d.nPad, c->held);
-    if (wide) {
-      p.binGroups = (d.n + BIN_GROUP_ATOMS - 1) / BIN_GROUP_ATOMS;
-      p.binTable = devAlloc<int>((size_t)p.binGroups * p.K[0], c->held);
-    }
+  } else if (!shared && p.K[0] >= PME_ORDER && (bins == 1 || (bins == 0 && d.n >= CELLS_SINGLE_MIN_ATOMS))) {
+    p.atoms = PME_ATOMS_CELLS;
   }
-  c->pmeBinned = p.binned;
+  c->pmeAtoms = p.atoms;
+  if (!p.planes) p.atoms = PME_ATOMS_CELLS;
   // A small single system folds its x lines into the plane gathers on
   // force-only evaluations (PmeDev::xFolded); the kernel X is kept whenever
   // the grid allows it, so the pipeline can be switched either way.
@@ -1356,7 +1350,7 @@ void create(rmd_ctx *c, const System &sys, const rmd_options &o, const Streams *
   p.xKernel = nullptr;
   if (!shared && p.K[0] <= X_FOLD_MAX_K) {
     p.xKernel = devAlloc<float>(2 * half, c->held);
-    p.xFolded = p.planes && !p.binned ? 1 : 0;
+    p.xFolded = p.planes && p.atoms == PME_ATOMS_SCAN ? 1 : 0;
   }
   c->pmeFolded = p.xFolded;
   writeBox(c);
@@ -2001,7 +1995,7 @@ int rmd_diagnostics_get(rmd_ctx *c, rmd_diagnostics *o) {
     o->pme_alpha = c->pme.alpha;
     o->lanes_per_atom = c->lanes;
     o->pme_planes = c->p.planes;
-    o->pme_x_folded = c->p.planes && c->p.xFolded && !c->p.binned ? 1 : 0;
+    o->pme_x_folded = c->p.planes && c->p.xFolded && c->p.atoms == PME_ATOMS_SCAN ? 1 : 0;
     o->water_units = c->waterUnits;
     o->cluster_units = c->clusterUnits;
     o->free_units = c->freeUnits;
@@ -2149,7 +2143,8 @@ int rmd_profile_kernel(rmd_ctx *c, int32_t kernel, int32_t reps, double *avg_ms)
         case 3: launchBonded(c->d, c->pme.alpha, RMD_TERM_ALL, 0, c->stream, nullptr); break;
         default:
           launchForceRebuildFlag(c->d, c->stream);
-          launchRebuild(c->d, c->stream);
+          launchCells(c->d, c->stream);
+          launchSearch(c->d, c->searchMode, c->stream);
           break;
       }
     };
@@ -2283,9 +2278,9 @@ int rmd_set_pme_pipeline(rmd_ctx *c, int32_t mode) {
       throw Error(RMD_E_INVALID, "one x plane of this PME grid does not fit in LDS");
     if (mode == PME_PLANES_FOLDED && !c->p.xKernel)
       throw Error(RMD_E_INVALID, "folded x lines need a single system of at most 32 x planes");
-    // planes without atom bins (every plane scans every atom), or the bins
-    // the context was created with; folded x lines as asked, or as created
-    c->p.binned = scan ? 0 : c->pmeBinned;
+    // planes that scan every atom, or find their atoms as the context was
+    // created to; the slabs go by cells; folded x lines as asked, or as created
+    c->p.atoms = scan ? PME_ATOMS_SCAN : c->p.planes ? c->pmeAtoms : PME_ATOMS_CELLS;
     c->p.xFolded = mode == PME_PLANES_FOLDED ? 1 : mode == PME_AUTO ? c->pmeFolded : 0;
     invalidateGraphs(c);
   });
@@ -2448,6 +2443,7 @@ void uploadViews(rmd_batch *b) {
     BatchView &v = b->views[r];
     v.d = c->d;
     v.p = c->p;
+    v.p.atoms = c->p.atoms == PME_ATOMS_CELLS ? c->pmeAtoms : c->p.atoms;  // (a batch has no slab pipeline)
     v.ip = c->ip;
     v.openBlocks = replicaBlocks(c, BK_OPEN);
     v.openSlots = openSlotCount(c->d);
@@ -2957,7 +2953,7 @@ void createBatch(rmd_batch *b, const rmd_system *const *systems, int count, cons
     if (!sys.positions.empty())
       setState(c, sys.positions.data(), sys.velocities.empty() ? nullptr : sys.velocities.data(), 0, 0);
     if (!c->p.planes)
-      throw Error(RMD_E_INVALID, replicaLabel(r) + "its PME grid needs the line pipeline, which a batch does not run");
+      throw Error(RMD_E_INVALID, replicaLabel(r) + "its PME grid needs the slab pipeline, which a batch does not run");
     if (!fitsSmallCellBuild(c->d.n, c->plan.cellCount))
       throw Error(RMD_E_INVALID, replicaLabel(r) + "a batch replica takes at most 16384 atoms and 4096 cells");
     if (r == 0)

@@ -59,6 +59,8 @@ struct Scalars {
   float slack;                // nm of the skin spent by volume moves since the last rebuild
   unsigned int spanBits;      // largest atom-to-centroid distance of any molecule seen (float bits)
   long long step;             // the noise counter (completed steps)
+  unsigned int cellTicket;    // last-block ticket of the cell assignment
+  unsigned int unused;
 };
 
 // A rebuild retires the current list's requirement into requiredMax before

@@ -9,12 +9,15 @@
 namespace rmd {
 
 // ---- cell list and neighbour list (neighbours.hip) ----
-// The five rebuild stages are launched every step and return at once unless
-// the integrator's last block (or the host) asked for a rebuild; with
-// `cellsBuilt` a small system's cell build is left out (the step's integrator
-// builds its cell list: IntegratorParams::cellsInIntegrator), with `searched`
-// the list search (the joined force launch runs it).
-void launchRebuild(const Dev &d, hipStream_t s, bool cellsBuilt = false, bool searched = false);
+// The cell list and the neighbour list, launched every step; every kernel
+// returns at once unless the integrator's last block (or the host) asked for
+// a rebuild. A small system's step leaves the cell build to its integrator
+// (IntegratorParams::cellsInIntegrator) and the search to its joined force
+// launch.
+void launchCells(const Dev &d, hipStream_t s);
+// mode: the context's search mode (1 by atom, 2 by cell where the launch
+// covers the cells, 0 by occupancy).
+void launchSearch(const Dev &d, int mode, hipStream_t s);
 void launchForceRebuildFlag(const Dev &d, hipStream_t s);
 
 // ---- nonbonded direct space (nonbonded.hip) ----
@@ -32,7 +35,6 @@ int launchBonded(const Dev &d, double alpha, int terms, int energies, hipStream_
 struct PmeDev {
   int K[3];
   int K2h;                  // K[2]/2 + 1
-  long long *qgrid;         // K0*K1*K2 fixed-point charges
   float2 *cgrid;            // K0*K1*K2h complex half spectrum
   float *rgrid;             // K0*K1*K2 real potential
   float *influence;         // K0*K1*K2h: pref * kernel(m) (0 at m = 0)
@@ -41,18 +43,13 @@ struct PmeDev {
   double piOverAlpha2;      // pi^2 / alpha^2 (the scaling derivative of the reciprocal energy)
   int planeSpan;            // max(ceil(K1/2) * K2, K2h * K1): one plane's complex work buffer
   int planeRegion;          // float2 slots of the second buffer: max(planeSpan, the int64 plane)
-  int planes;               // 1: plane pipeline, 0: line pipeline
-  // The plane pipeline's atoms by the base index of their x support (K0
-  // bins): a plane reads the ORDER bins that reach it instead of every atom.
-  int binned;               // 1: the bins are built each evaluation (replica batches, large systems)
-  int *binStart;            // K0 + 1 offsets into binAtoms
+  int planes;               // 1: plane pipeline, 0: slab pipeline
+  int slabLines[3];         // slab pipeline: lines per LDS tile of each axis' pass
+  // How a plane finds the atoms that reach it; see PME_ATOMS_*.
+  int atoms;
+  int *binStart;            // bins: K0 + 1 offsets into binAtoms
   int2 *atomBin;            // per atom: (bin or -1 for no charge, rank in the bin)
   int *binAtoms;            // atoms grouped by bin
-  // A large single system builds its bins in three launches over groups of
-  // BIN_GROUP_ATOMS atoms (binGroups > 0): per-group counts, their offsets,
-  // the scatter. 0: one workgroup builds them (batch members).
-  int binGroups;
-  int *binTable;            // K0 x binGroups counts, then offsets within each bin
   // A small single system's force-only evaluations fold the x lines into the
   // plane gathers: the forward x transform, the influence function and the
   // inverse x transform of every (y, z) column are one circular convolution
@@ -67,6 +64,14 @@ struct PmeDev {
   int xReal;                // 1: X is real (a rectangular box, where g is even in k)
   float *xKernel;           // X as K0 x (K1 * K2h) floats (xReal) or float2s; null when not allocated
 };
+// SCAN: every plane scans every atom (small single systems, whose cells are
+// as wide as the box; no launch and no dependency of its own). CELLS: a plane
+// scans the slots of the cells its support can come from, a run of the cell
+// order (larger single systems; the cell list first). BINS: the atoms are
+// binned by the base index of their x support in a launch of its own, one
+// workgroup per system (batch members, whose cells are few and whose launches
+// are shared).
+enum { PME_ATOMS_SCAN = 0, PME_ATOMS_BINS = 1, PME_ATOMS_CELLS = 2 };
 // Grids up to this many x planes may fold their x lines into the gathers
 // (each gather workgroup reads all K0 forward planes and K0 kernel rows).
 constexpr int X_FOLD_MAX_K = 32;
@@ -77,12 +82,9 @@ bool pmeConfigure(PmeDev &p, int mode, size_t maxLds);
 // Whether a plane-pipeline system can bin its atoms in one workgroup.
 constexpr int BIN_MAX_ATOMS = 16384;
 bool pmeBinsFit(const PmeDev &p, int atoms);
-// Single systems of at least this many atoms bin their plane-pipeline atoms
-// (smaller ones scan every atom per plane: one launch fewer on a short
-// critical path), in groups of BIN_GROUP_ATOMS.
-constexpr int BIN_SINGLE_MIN_ATOMS = 8192;
-constexpr int BIN_GROUP_ATOMS = 1024;
-bool pmeBinsFitWide(const PmeDev &p);
+// Single systems of at least this many atoms look for a plane's atoms by
+// cells (smaller ones scan every atom per plane).
+constexpr int CELLS_SINGLE_MIN_ATOMS = 8192;
 // The device box set from its value and the influence function computed from
 // it, in one launch (then the folded x lines' kernel where it is kept).
 void pmeSetBoxAndInfluence(const PmeDev &p, const BoxF &box, BoxF *dst, const double *moduli[3], double alpha,
@@ -96,7 +98,7 @@ int launchPme(const Dev &d, const PmeDev &p, int energies, hipStream_t s, int *s
 // launchPmeAfterForward then runs the rest of the plane pipeline and returns
 // its slots. With `search` (the one-wave-per-atom list search) a rebuild's
 // list search runs there too: each direct-space workgroup searches its own
-// rows before it computes them, and launchRebuild leaves its search out.
+// rows before it computes them (no launchSearch).
 bool forcesJoin(const Dev &d, const PmeDev &p, int lanes);
 void launchForcesJoined(const Dev &d, const PmeDev &p, float alpha, int rational, int lanes, int energies,
                         double alphaD, int terms, hipStream_t s, int *pairSlots, int *bondedSlots, int search = 0);

@@ -29,38 +29,53 @@ __global__ void setRebuildKernel(Scalars *sc) {
   sc->rebuilds += 1u;
 }
 
-__global__ void cellsAssignKernel(Dev d) {
-  if (!d.sc->rebuild) return;
-  const BoxF &box = *d.box;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= d.n) return;
-  const float4 p = d.pos[i];
-  int c3[3];
-  const int c = cellIndex(p.x, p.y, p.z, box, c3);
-  d.cellOfAtom[i] = c;
-  atomicAdd(&d.cellCount[c], 1);
-  if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) atomicMax(&d.sc->nonFinite, 1u);
-}
-
-// Exclusive scan of the per-cell counts in one workgroup, SCAN_TILE cells at
-// a time. A tile's counts are loaded coalesced into LDS, every load of a
-// thread in flight together (a thread reading its own contiguous run from
-// global memory waited one full latency per cell). Each thread then sums its
-// run of SCAN_RUN cells in LDS; the runs' sums are scanned across the
-// workgroup; each thread writes its run's starts back to LDS; the tile's
-// starts go out coalesced. Leaves the counts zeroed for the next rebuild and
-// the scatter cursors at the cell starts.
+// A large system's cell list is three launches, which return at once on the
+// steps that keep it: the assignment with the scan, the scatter, the sort of
+// each cell. They come before the PME and direct-space branches fork, so
+// every step pays for them: five launches, the scan and the long cells' sort
+// by themselves, made a step of 24,022 atoms 8 us longer.
+//
+// 1. Each atom's cell, counted; then the last workgroup to finish scans the
+// counts, exclusive, SCAN_TILE cells at a time. A tile's counts are loaded
+// coalesced into LDS, every load of a thread in flight together (a thread
+// reading its own contiguous run from global memory waited one full latency
+// per cell). Each thread then sums its run of SCAN_RUN cells in LDS; the
+// runs' sums are scanned across the workgroup; each thread writes its run's
+// starts back to LDS; the tile's starts go out coalesced. Leaves the counts
+// zeroed for the next rebuild and the scatter cursors at the cell starts.
 constexpr int SCAN_THREADS = 1024, SCAN_RUN = 8, SCAN_TILE = SCAN_THREADS * SCAN_RUN;
 
 // LDS index of tile entry k, one pad word per 32 so the threads' runs start
 // in different banks
 __device__ __forceinline__ int scanPad(int k) { return k + (k >> 5); }
 
-__global__ void __launch_bounds__(SCAN_THREADS) cellsScanKernel(Dev d) {
+__global__ void __launch_bounds__(SCAN_THREADS) cellsAssignKernel(Dev d) {
   if (!d.sc->rebuild) return;
   __shared__ int tile[SCAN_TILE + SCAN_TILE / 32];
   __shared__ int partial[SCAN_THREADS];
-  const int total = d.box->cellTotal, t = threadIdx.x;
+  __shared__ bool last;
+  const int t = threadIdx.x;
+  {
+    const BoxF &box = *d.box;
+    const int i = blockIdx.x * SCAN_THREADS + t;
+    if (i < d.n) {
+      const float4 p = d.pos[i];
+      int c3[3];
+      const int c = cellIndex(p.x, p.y, p.z, box, c3);
+      d.cellOfAtom[i] = c;
+      atomicAdd(&d.cellCount[c], 1);
+      if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z))) atomicMax(&d.sc->nonFinite, 1u);
+    }
+  }
+  // every workgroup's counts are released before its ticket; the last one
+  // acquires them and reads them past the caches
+  __threadfence();
+  __syncthreads();
+  if (t == 0) last = atomicAdd(&d.sc->cellTicket, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  const int total = d.box->cellTotal;
   int carry = 0;
   for (int base = 0; base < total; base += SCAN_TILE) {
     const int here = min(SCAN_TILE, total - base);
@@ -68,7 +83,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) cellsScanKernel(Dev d) {
 #pragma unroll
     for (int u = 0; u < SCAN_RUN; ++u) {
       const int k = t + SCAN_THREADS * u;
-      v[u] = k < here ? d.cellCount[base + k] : 0;
+      v[u] = k < here ? __hip_atomic_load(&d.cellCount[base + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
     }
 #pragma unroll
     for (int u = 0; u < SCAN_RUN; ++u) tile[scanPad(t + SCAN_THREADS * u)] = v[u];
@@ -107,7 +122,10 @@ __global__ void __launch_bounds__(SCAN_THREADS) cellsScanKernel(Dev d) {
     carry += tileTotal;
     __syncthreads();  // the next tile reuses tile and partial
   }
-  if (t == 0) d.cellStart[total] = carry;
+  if (t == 0) {
+    d.cellStart[total] = carry;
+    d.sc->cellTicket = 0u;
+  }
 }
 
 __global__ void cellsScatterKernel(Dev d) {
@@ -121,66 +139,64 @@ __global__ void cellsScatterKernel(Dev d) {
 // The scatter leaves each cell's atoms in arrival order; sorting each cell's
 // run puts them in index order so the list, and every sum over it, is the
 // same on every run. Sorted cells also get their slots written (positions in
-// cell order, with the atom index in .w, for the candidate scan). Cells of at
-// most SHORT_CELL atoms - every cell of a plan whose cells are a fraction of
-// the list cutoff - are sorted by one thread each, by insertion in that
-// thread's slice of LDS; longer ones by a bitonic sort over a workgroup
-// (cellsSortLongKernel).
+// cell order, with the atom index in .w, for the candidate scan). A workgroup
+// takes CELLS_PER_SORT cells: those of at most SHORT_CELL atoms - every cell
+// of a plan whose cells are a fraction of the list cutoff - are sorted by one
+// thread each, by insertion in that thread's slice of LDS; longer ones then
+// by a bitonic sort over the workgroup, in the same LDS.
 constexpr int SHORT_CELL = 32;
-constexpr int SHORT_SORT_THREADS = 128;
+constexpr int CELLS_PER_SORT = 128;
 
-__global__ void __launch_bounds__(SHORT_SORT_THREADS) cellsSortShortKernel(Dev d) {
+__global__ void __launch_bounds__(CELLS_PER_SORT) cellsSortKernel(Dev d) {
   if (!d.sc->rebuild) return;
-  __shared__ int keys[SHORT_SORT_THREADS][SHORT_CELL + 1];  // +1: the threads' slices start in different banks
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= d.box->cellTotal) return;
-  const int begin = d.cellStart[c], len = d.cellStart[c + 1] - begin;
-  if (len > SHORT_CELL) return;
-  int *k = keys[threadIdx.x];
-  // the cell's atoms loaded together, then sorted in LDS
-  for (int a = 0; a < len; ++a) k[a] = d.cellAtoms[begin + a];
-  for (int a = 1; a < len; ++a) {
-    const int v = k[a];
-    int m = a - 1;
-    while (m >= 0 && k[m] > v) {
-      k[m + 1] = k[m];
-      --m;
+  // +1: the threads' slices start in different banks
+  constexpr int SLICE = SHORT_CELL + 1;
+  __shared__ int keys[CELLS_PER_SORT * SLICE > SORT_CAPACITY ? CELLS_PER_SORT * SLICE : SORT_CAPACITY];
+  const int total = d.box->cellTotal, first = blockIdx.x * CELLS_PER_SORT;
+  const int c = first + threadIdx.x;
+  const int begin = c < total ? d.cellStart[c] : 0, len = c < total ? d.cellStart[c + 1] - begin : 0;
+  if (len <= SHORT_CELL) {
+    int *k = keys + threadIdx.x * SLICE;
+    // the cell's atoms loaded together, then sorted in LDS
+    for (int a = 0; a < len; ++a) k[a] = d.cellAtoms[begin + a];
+    for (int a = 1; a < len; ++a) {
+      const int v = k[a];
+      int m = a - 1;
+      while (m >= 0 && k[m] > v) {
+        k[m + 1] = k[m];
+        --m;
+      }
+      k[m + 1] = v;
     }
-    k[m + 1] = v;
-  }
-  // positions and types SLOT_BATCH at a time, loaded before any slot is
-  // written (a slot's stores would otherwise wait on its own loads, one
-  // round trip per atom)
-  constexpr int SLOT_BATCH = 4;
-  for (int a = 0; a < len; a += SLOT_BATCH) {
-    float4 p[SLOT_BATCH];
-    int type[SLOT_BATCH];
+    // positions and types SLOT_BATCH at a time, loaded before any slot is
+    // written (a slot's stores would otherwise wait on its own loads, one
+    // round trip per atom)
+    constexpr int SLOT_BATCH = 4;
+    for (int a = 0; a < len; a += SLOT_BATCH) {
+      float4 p[SLOT_BATCH];
+      int type[SLOT_BATCH];
 #pragma unroll
-    for (int u = 0; u < SLOT_BATCH; ++u) {
-      const int atom = k[min(a + u, len - 1)];
-      p[u] = d.pos[atom];
-      type[u] = d.type[atom];
+      for (int u = 0; u < SLOT_BATCH; ++u) {
+        const int atom = k[min(a + u, len - 1)];
+        p[u] = d.pos[atom];
+        type[u] = d.type[atom];
+      }
+#pragma unroll
+      for (int u = 0; u < SLOT_BATCH; ++u)
+        if (a + u < len) writeSlotLoaded(d, begin + a + u, k[a + u], p[u], type[u]);
     }
-#pragma unroll
-    for (int u = 0; u < SLOT_BATCH; ++u)
-      if (a + u < len) writeSlotLoaded(d, begin + a + u, k[a + u], p[u], type[u]);
   }
-}
-
-__global__ void __launch_bounds__(256) cellsSortLongKernel(Dev d) {
-  if (!d.sc->rebuild) return;
-  __shared__ int keys[SORT_CAPACITY];
-  for (int c = blockIdx.x; c < d.box->cellTotal; c += gridDim.x) {
-    const int begin = d.cellStart[c], end = d.cellStart[c + 1];
-    const int len = end - begin;
-    if (len <= SHORT_CELL) continue;
-    if (len > SORT_CAPACITY) {
+  if (!__syncthreads_or(len > SHORT_CELL)) return;
+  for (int q = first; q < min(total, first + CELLS_PER_SORT); ++q) {
+    const int b = d.cellStart[q], n = d.cellStart[q + 1] - b;
+    if (n <= SHORT_CELL) continue;
+    if (n > SORT_CAPACITY) {
       if (threadIdx.x == 0) atomicMax(&d.sc->cellOverflow, 1u);
       continue;
     }
     int size = 1;
-    while (size < len) size <<= 1;
-    for (int k = threadIdx.x; k < size; k += blockDim.x) keys[k] = k < len ? d.cellAtoms[begin + k] : 0x7fffffff;
+    while (size < n) size <<= 1;
+    for (int k = threadIdx.x; k < size; k += blockDim.x) keys[k] = k < n ? d.cellAtoms[b + k] : 0x7fffffff;
     __syncthreads();
     for (int k = 2; k <= size; k <<= 1) {
       for (int j = k >> 1; j > 0; j >>= 1) {
@@ -188,17 +204,17 @@ __global__ void __launch_bounds__(256) cellsSortLongKernel(Dev d) {
           const int partner = t ^ j;
           if (partner > t) {
             const bool ascending = (t & k) == 0;
-            const int a = keys[t], b = keys[partner];
-            if ((a > b) == ascending) {
-              keys[t] = b;
-              keys[partner] = a;
+            const int x = keys[t], y = keys[partner];
+            if ((x > y) == ascending) {
+              keys[t] = y;
+              keys[partner] = x;
             }
           }
         }
         __syncthreads();
       }
     }
-    for (int k = threadIdx.x; k < len; k += blockDim.x) writeSlot(d, begin + k, keys[k]);
+    for (int k = threadIdx.x; k < n; k += blockDim.x) writeSlot(d, b + k, keys[k]);
     __syncthreads();  // keys is reused for the workgroup's next cell
   }
 }
@@ -416,22 +432,32 @@ bool integratorBuildsCells(const Dev &d, int cellCount) {
   return d.n <= SMALL_MAX_ATOMS && d.cellCapacity <= SMALL_MAX_CELLS && cellCount <= FEW_MAX_CELLS && !splitWater(d);
 }
 
-void launchRebuild(const Dev &d, hipStream_t s, bool cellsBuilt, bool searched) {
+void launchCells(const Dev &d, hipStream_t s) {
   if (d.n <= SMALL_MAX_ATOMS && d.cellCapacity <= SMALL_MAX_CELLS) {
-    if (!cellsBuilt) cellsBuildSmallKernel<<<1, SMALL_THREADS, 0, s>>>(d);
-  } else {
-    const int blocks = (d.n + 255) / 256;
-    cellsAssignKernel<<<blocks, 256, 0, s>>>(d);
-    cellsScanKernel<<<1, SCAN_THREADS, 0, s>>>(d);
-    cellsScatterKernel<<<blocks, 256, 0, s>>>(d);
-    cellsSortShortKernel<<<(d.cellCapacity + SHORT_SORT_THREADS - 1) / SHORT_SORT_THREADS, SHORT_SORT_THREADS, 0, s>>>(d);
-    cellsSortLongKernel<<<std::min(d.cellCapacity, 1024), 256, 0, s>>>(d);
+    cellsBuildSmallKernel<<<1, SMALL_THREADS, 0, s>>>(d);
+    return;
   }
-  if (searched) return;
+  cellsAssignKernel<<<(d.n + SCAN_THREADS - 1) / SCAN_THREADS, SCAN_THREADS, 0, s>>>(d);
+  cellsScatterKernel<<<(d.n + 255) / 256, 256, 0, s>>>(d);
+  cellsSortKernel<<<(d.cellCapacity + CELLS_PER_SORT - 1) / CELLS_PER_SORT, CELLS_PER_SORT, 0, s>>>(d);
+}
+
+// The per-cell search runs in the per-atom search's launch (4 waves per
+// workgroup, one workgroup per 4 atoms), so it covers at most that many cells.
+static bool cellLaunchCovers(int atoms, int cells) { return cells > 0 && cells <= 4 * ((atoms + 3) / 4); }
+
+// One workgroup per four atoms covers either form of the search. Where every
+// plan the cell arrays can hold is searched by cell (mode 2, at most one cell
+// per atom of the launch), one per four cells does, and the steps that keep
+// the list end sooner: 100,200 atoms in 17,576 cells, 25,050 workgroups that
+// return at once took 5.6 us of each step.
+void launchSearch(const Dev &d, int mode, hipStream_t s) {
+  const bool byCell = mode == 2 && cellLaunchCovers(d.n, d.cellCapacity);
+  const int blocks = ((byCell ? d.cellCapacity : d.n) + 3) / 4;
   if (d.rect)
-    neighboursKernel<true><<<(d.n + 3) / 4, 256, 0, s>>>(d);
+    neighboursKernel<true><<<blocks, 256, 0, s>>>(d);
   else
-    neighboursKernel<false><<<(d.n + 3) / 4, 256, 0, s>>>(d);
+    neighboursKernel<false><<<blocks, 256, 0, s>>>(d);
 }
 
 // Batched rebuild: every replica's cell list in one workgroup of its own (a
@@ -451,10 +477,6 @@ void launchRebuildBatch(const BatchView *v, const TaskTable &replicaTable, int r
 int searchQueueInts(int replicas) { return 3 + 2 * replicas; }
 
 bool fitsSmallCellBuild(int atoms, int cells) { return atoms <= SMALL_MAX_ATOMS && cells <= SMALL_MAX_CELLS; }
-
-// The per-cell search runs in the per-atom search's launch (4 waves per
-// workgroup, one workgroup per 4 atoms), so it covers at most that many cells.
-static bool cellLaunchCovers(int atoms, int cells) { return cells > 0 && cells <= 4 * ((atoms + 3) / 4); }
 
 bool cellSearchFits(int atoms, int cells) {
   constexpr int MAX_AVERAGE = 32;  // atoms per cell

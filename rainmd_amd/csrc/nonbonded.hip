@@ -387,11 +387,11 @@ int launchNonbonded(const Dev &d, float alpha, int rational, int lanes, int ener
 // VGPRs against the direct space's 63 at 64 lanes): a system joins when its
 // direct space fits in one pass at four waves per SIMD of the 256 CUs, as
 // small systems' launch-bound steps do, with the LJ table in LDS, the
-// unbinned plane pipeline and at most 64 KB of LDS per workgroup.
+// plane pipeline scanning every atom and at most 64 KB of LDS per workgroup.
 bool forcesJoin(const Dev &d, const PmeDev &p, int lanes) {
   constexpr long long ONE_PASS = 256LL * 4 * 4 * 64;  // threads
   return (lanes == 16 || lanes == 32 || lanes == 64) && (long long)d.n * lanes <= ONE_PASS && tableInLds(d.types) &&
-         p.planes && !p.binned && std::max(tableLdsBytes(d.types), pmePlaneForwardLds(p)) <= 65536;
+         p.planes && p.atoms == PME_ATOMS_SCAN && std::max(tableLdsBytes(d.types), pmePlaneForwardLds(p)) <= 65536;
 }
 
 void launchForcesJoined(const Dev &d, const PmeDev &p, float alpha, int rational, int lanes, int energies,

@@ -19,7 +19,6 @@ constexpr int ORDER = 5;
 constexpr int PLANE_THREADS = 512;
 constexpr int XLINE_THREADS = PLANE_THREADS;  // the x lines run in the plane kernels' workgroup shape
 constexpr int XLINES = 16;                     // x lines per workgroup in the plane pipeline
-constexpr int LINES_PER_BLOCK = 4;  // lines per workgroup in the line pipeline
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
@@ -91,6 +90,19 @@ __device__ __forceinline__ void smallDft(float2 *v, int R, int sign) {
   }
 }
 
+// Division of a non-negative index by an axis length or a line count the same
+// for a whole launch: the grid's sizes are known only at run time, and an
+// integer division by such a divisor is some forty instructions, two of them
+// per butterfly. (i + 1/2) * (1 / d) in FP32 is off by less than 1e-6 of
+// itself and at least 1 / 2d from an integer, so the truncation is exact for
+// i < 2^19 (a plane of 725^2; LDS ends long before).
+struct Div {
+  int d;
+  float inv;
+  __device__ __forceinline__ explicit Div(int divisor) : d(divisor), inv(1.0f / (float)divisor) {}
+  __device__ __forceinline__ int operator()(int i) const { return (int)(((float)i + 0.5f) * inv); }
+};
+
 // One radix-R pass of a Stockham autosort FFT over `lines` lines of length K
 // (line l at src + l * K, in LDS); `Ns` is the product of the radices done.
 // R is a compile-time constant, so the butterfly stays in registers.
@@ -98,13 +110,14 @@ template <int R>
 __device__ __forceinline__ void fftStage(const float2 *src, float2 *dst, int lines, int K, int Ns, const float2 *tw,
                                          int sign) {
   const int L = K / R;
-  const int twStride = K / (Ns * R);
+  const Div byL(L), byNs(Ns);
+  const int twStride = byNs(L);
   const int total = lines * L;
   for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-    const int line = idx / L, j = idx - line * L;
+    const int line = byL(idx), j = idx - line * L;
     const float2 *in = src + line * K;
     float2 *out = dst + line * K;
-    const int k = j % Ns;
+    const int q0 = byNs(j), k = j - q0 * Ns;
     float2 v[8];
     v[0] = in[j];
 #pragma unroll
@@ -114,7 +127,7 @@ __device__ __forceinline__ void fftStage(const float2 *src, float2 *dst, int lin
       v[q] = cmul(in[j + q * L], w);
     }
     smallDft(v, R, sign);
-    const int base = (j / Ns) * Ns * R + k;
+    const int base = q0 * Ns * R + k;
 #pragma unroll
     for (int q = 0; q < R; ++q) out[base + q * Ns] = v[q];
   }
@@ -200,20 +213,34 @@ __device__ __forceinline__ void gridCoordinate(const PmeDev &p, const double *re
   offset = (float)off;
 }
 
-// Grid index of weight k for base b: (b + k - order + 1) mod K.
+// Grid index of weight k for base b: (b + k - order + 1) mod K (K >= ORDER:
+// the host refuses smaller grids, so one addition wraps it).
 __device__ __forceinline__ int gridIndex(int b, int k, int K) {
-  int g = b + k - (ORDER - 1);
-  while (g < 0) g += K;
-  while (g >= K) g -= K;
-  return g;
+  const int g = b + k - (ORDER - 1);
+  return g < 0 ? g + K : g;
 }
 
-// The first weight index k with gridIndex(b, k, K) == plane, or ORDER if the
-// atom's support misses the plane (later matches are k + K, k + 2K, ...).
+// The weight index k with gridIndex(b, k, K) == plane, or at least ORDER if
+// the atom's support misses the plane.
 __device__ __forceinline__ int planeWeight(int b, int plane, int K) {
-  int r = (plane - b + ORDER - 1) % K;
-  if (r < 0) r += K;
-  return r;
+  int r = plane - b + ORDER - 1;
+  r += r < 0 ? K : 0;
+  return r >= K ? r - K : r;
+}
+
+// Whether a position's support may reach grid points [first, first + points)
+// of an axis, in FP32 on the safe side: the fractional coordinate's rounding
+// stays far below the margin of 1/16 grid point for positions within 64 boxes
+// of the origin and K <= 1024, and further positions pass. A quarter of the
+// exact test's time (gridCoordinate in FP64), which the few that pass still
+// take.
+__device__ __forceinline__ bool mayReach(const float r[3], int K, int first, int points, float4 pos) {
+  const float f = pos.x * r[0] + pos.y * r[1] + pos.z * r[2];
+  const float k = (float)K, margin = 0.0625f;
+  float u = (f - floorf(f)) * k - ((float)first - margin);  // past the first base index
+  u -= u >= k ? k : 0.f;
+  u += u < 0.f ? k : 0.f;
+  return u <= (float)(points + ORDER - 1) + 2.0f * margin || !(fabsf(f) < 64.0f);
 }
 
 // round-to-nearest-even of v to an integer, exact for |v| < 2^51: adding
@@ -303,13 +330,95 @@ __device__ __forceinline__ void planeRanges(const PmeDev &p, int i, int2 range[2
   }
 }
 
-// One round of a plane's atom scan: of atoms [a0, a0 + PLANE_THREADS * SCAN),
-// those whose x support meets `plane` are appended to `list` as 16 bits,
-// (atom - a0) << 3 | weight index, wave-aggregated into the shared `count`.
-// The expensive per-atom work then runs over the compacted list with every
-// lane busy (about 5 in K0 atoms land on a given plane). Single systems scan
-// six atoms per thread: a 3,072-atom system in one round (each round is a
-// global-load latency and three barriers on the kernel's serial path), in
+// The cells along `axis` that an atom whose support touches grid points
+// [first, first + points) of that axis can have been assigned to at the last
+// rebuild: its base index lies in [first, first + points + ORDER - 2], and it
+// has moved by at most half the skin since (what volume moves spend of the
+// skin included). `start` in [0, cells), `count` at most cells; the run may
+// wrap. The margin's last terms are far above the rounding of the FP32 cell
+// assignment.
+__device__ __forceinline__ void supportCells(const Dev &d, int axis, int first, int points, int K, int &start,
+                                             int &count) {
+  const BoxF &b = *d.box;
+  const int cells = b.cells[axis];
+  const float moved = 0.5f * (sqrtf(b.rl2) - b.cutoff) + 1e-3f;
+  const float r0 = b.recip[axis], r1 = b.recip[3 + axis], r2 = b.recip[6 + axis];
+  const float margin = moved * sqrtf(r0 * r0 + r1 * r1 + r2 * r2) + 2e-5f;
+  const float lo = (float)first / (float)K - margin, hi = (float)(first + points + ORDER - 1) / (float)K + margin;
+  const int c0 = (int)floorf(lo * (float)cells), c1 = (int)floorf(hi * (float)cells);
+  if (c1 - c0 + 1 >= cells) {
+    start = 0;
+    count = cells;
+    return;
+  }
+  count = c1 - c0 + 1;
+  start = c0 % cells;
+  start += start < 0 ? cells : 0;
+}
+
+// The slots a plane's atoms can be in: one run of the cell order (x slowest)
+// or two where it wraps.
+__device__ __forceinline__ void planeSlots(const Dev &d, const PmeDev &p, int i, int2 range[2]) {
+  const int cx = d.box->cells[0], slab = d.box->cells[1] * d.box->cells[2];
+  int start, count;
+  supportCells(d, 0, i, 1, p.K[0], start, count);
+  const int end = start + count;
+  range[0] = make_int2(d.cellStart[start * slab], d.cellStart[min(end, cx) * slab]);
+  range[1] = end > cx ? make_int2(d.cellStart[0], d.cellStart[(end - cx) * slab]) : make_int2(0, 0);
+}
+
+// Candidates tested one per lane and those that pass `test` acted on 64 at a
+// time: each wave takes every waves-th chunk of `total` candidates, keeps the
+// hits in a queue of its own in LDS and empties it whenever it holds a whole
+// wave of them. No barrier inside: a workgroup's waves hide each other's
+// loads, where rounds of a list shared by the workgroup (three barriers each)
+// waited for every wave's. map(g) is candidate g's entry, pos(entry) its
+// position. The queue holds QUEUE_CAND + 1 waves of entries.
+constexpr int QUEUE_CAND = 3;  // candidates per lane in flight
+constexpr int QUEUE_ENTRIES = 64 * (QUEUE_CAND + 1);
+
+template <typename E, typename Map, typename Pos, typename Test, typename Act>
+__device__ __forceinline__ void waveQueue(int total, E *queues, Map map, Pos pos, Test test, Act act) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  E *queue = queues + wave * QUEUE_ENTRIES;
+  int held = 0;
+  for (int base = wave * 64 * QUEUE_CAND; base < total; base += waves * 64 * QUEUE_CAND) {
+    E entry[QUEUE_CAND];
+    float4 at[QUEUE_CAND];
+#pragma unroll
+    for (int u = 0; u < QUEUE_CAND; ++u) {
+      const int g = base + u * 64 + lane;
+      entry[u] = 0;
+      at[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (g < total) {
+        entry[u] = map(g);
+        at[u] = pos(entry[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < QUEUE_CAND; ++u) {
+      const bool take = test(at[u]);
+      const unsigned long long mask = __ballot(take);
+      if (take) queue[held + __popcll(mask & ((1ull << lane) - 1ull))] = entry[u];
+      held += __popcll(mask);
+    }
+    __builtin_amdgcn_wave_barrier();
+    while (held >= 64) {
+      held -= 64;
+      act(pos(queue[held + lane]));
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (lane < held) act(pos(queue[lane]));
+}
+
+// One round of a plane's scan of every atom: of atoms [a0, a0 + threads *
+// SCAN), those whose x support meets `plane` are appended to `list` as 16
+// bits, (atom - a0) << 3 | weight index, wave-aggregated into the shared
+// `count`. The expensive per-atom work then runs over the compacted list with
+// every lane busy (about 5 in K0 atoms land on a given plane). Single systems
+// scan six atoms per thread: a 3,072-atom system in one round (each round is
+// a global-load latency and three barriers on the kernel's serial path), in
 // less LDS than 2,048 int entries. The batched kernels scan four: their
 // members mostly take the binned path, and the wider scan's registers would
 // cost them a workgroup per CU.
@@ -361,8 +470,6 @@ __device__ void planeScan(const Dev &d, const PmeDev &p, int plane, int a0, Plan
   planeScanTake<SCAN>(d, p, plane, a0, batch, list, count);
 }
 
-
-
 // 1. Spread onto plane i and forward z, y transforms of the plane. With
 // `real` set, the plane is read from a real K0*K1*K2 grid instead (the FFT
 // verification entry).
@@ -370,6 +477,7 @@ template <int SCAN = SCAN_PER_THREAD>
 __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, const float *real, int i, float2 *lds) {
   const int K0 = p.K[0], K1 = p.K[1], K2 = p.K[2], K2h = p.K2h;
   const int S = p.planeSpan, P = (K1 + 1) / 2;
+  const Div byK1(K1), byK2(K2), byK2h(K2h);
   const int t = threadIdx.x, nt = blockDim.x;
   float2 *tw1 = lds, *tw2 = tw1 + K1;
   float2 *A = tw2 + K2, *B = A + S;
@@ -377,37 +485,36 @@ __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, c
   PlaneEntry *list = reinterpret_cast<PlaneEntry *>(B + p.planeRegion);
   int *listCount = reinterpret_cast<int *>(list + PLANE_LIST);
   // the first scan round's positions, in flight with the twiddles' loads
-  const bool scanning = !real && !p.binned;
+  const bool scanning = !real && p.atoms == PME_ATOMS_SCAN;
   float4 first[SCAN];
   if (scanning) planeScanLoad<SCAN>(d, 0, first);
   loadTwiddles(tw1, p.twiddle[1], K1);
   loadTwiddles(tw2, p.twiddle[2], K2);
   if (real) {
     for (int idx = t; idx < P * K2; idx += nt) {
-      const int pr = idx / K2, k = idx - pr * K2;
+      const int pr = byK2(idx), k = idx - pr * K2;
       const float *row = real + ((size_t)i * K1 + 2 * pr) * K2;
       A[idx] = make_float2(row[k], 2 * pr + 1 < K1 ? row[K2 + k] : 0.f);
     }
   } else {
     for (int idx = t; idx < K1 * K2; idx += nt) plane[idx] = 0;
     const double *recip = d.box->recip64;
-    // atom a's charge onto this plane; r: the first weight index that lands
-    // on the plane, or -1 to derive it from a binned atom's base index (in
-    // i .. i + ORDER - 1 mod K0)
-    auto spread = [&](int a, int r) {
-      const float4 pos = d.pos[a];
+    // an atom's charge onto this plane; r: the first weight index that lands
+    // on the plane, or -1 to derive it (and to pass over an atom that only
+    // came near)
+    auto spread = [&](float4 pos, int r) {
       int bx, by, bz;
       float ox, oy, oz;
       gridCoordinate(p, recip, 0, pos, bx, ox);
       if (r < 0) {
-        r = i - bx + ORDER - 1;
-        r += r < 0 ? K0 : 0;
-        r -= r >= K0 ? K0 : 0;
+        r = planeWeight(bx, i, K0);
+        if (r >= ORDER) return;
       }
       float w[ORDER], wy[ORDER], wz[ORDER], dw[ORDER];
       bspline5(ox, w, dw);
-      float wx = 0.f;
-      for (int q = r; q < ORDER; q += K0) wx += w[q];
+      float wx = 0.f;  // (K0 >= ORDER: one weight lands on the plane)
+#pragma unroll
+      for (int q = 0; q < ORDER; ++q) wx = q == r ? w[q] : wx;
       gridCoordinate(p, recip, 1, pos, by, oy);
       gridCoordinate(p, recip, 2, pos, bz, oz);
       bspline5(oy, wy, dw);
@@ -421,11 +528,29 @@ __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, c
       }
     };
     __syncthreads();
-    if (p.binned) {
+    if (p.atoms == PME_ATOMS_CELLS) {
+      // queue entries are 16-bit candidate numbers, so the candidates go by
+      // in stretches of 65,536
+      const float recip32[3] = {(float)recip[0], (float)recip[3], (float)recip[6]};
+      int2 range[2];
+      planeSlots(d, p, i, range);
+      const int len = range[0].y - range[0].x, total = len + range[1].y - range[1].x;
+      for (int from = 0; from < total; from += 65536) {
+        auto slotOf = [&](int e) {
+          const int g = from + e;
+          return g < len ? range[0].x + g : range[1].x + (g - len);
+        };
+        waveQueue(
+            min(65536, total - from), list, [](int g) { return (PlaneEntry)g; },
+            [&](PlaneEntry e) { return d.slotPos[slotOf(e)]; },
+            [&](float4 pos) { return pos.w != 0.f && mayReach(recip32, K0, i, 1, pos); },
+            [&](float4 pos) { spread(pos, -1); });
+      }
+    } else if (!scanning) {
       int2 range[2];
       planeRanges(p, i, range);
       for (int h = 0; h < 2; ++h)
-        for (int k = range[h].x + t; k < range[h].y; k += nt) spread(p.binAtoms[k], -1);
+        for (int k = range[h].x + t; k < range[h].y; k += nt) spread(d.pos[p.binAtoms[k]], -1);
     } else {
       for (int a0 = 0; a0 < d.n; a0 += nt * SCAN) {
         if (t == 0) *listCount = 0;
@@ -436,14 +561,14 @@ __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, c
           planeScan<SCAN>(d, p, i, a0, list, listCount);
         __syncthreads();
         const int count = *listCount;
-        for (int k = t; k < count; k += nt) spread(a0 + (list[k] >> 3), list[k] & 7);
+        for (int k = t; k < count; k += nt) spread(d.pos[a0 + (list[k] >> 3)], list[k] & 7);
         __syncthreads();
       }
     }
     __syncthreads();
     // Two real z lines per complex line.
     for (int idx = t; idx < P * K2; idx += nt) {
-      const int pr = idx / K2, k = idx - pr * K2;
+      const int pr = byK2(idx), k = idx - pr * K2;
       const long long *row = plane + 2 * pr * K2;
       const float re = (float)((double)row[k] * GRID_UNSCALE);
       const float im = 2 * pr + 1 < K1 ? (float)((double)row[K2 + k] * GRID_UNSCALE) : 0.f;
@@ -456,7 +581,7 @@ __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, c
   // Split the packed spectra: line 2p = (Z[m] + conj Z[-m]) / 2, line 2p+1 =
   // (Z[m] - conj Z[-m]) / (2i); y lines laid out m-major.
   for (int idx = t; idx < K2h * K1; idx += nt) {
-    const int m = idx / K1, j = idx - m * K1;
+    const int m = byK1(idx), j = idx - m * K1;
     const float2 *zl = Z + (j >> 1) * K2;
     const float2 z = zl[m], zc = zl[m == 0 ? 0 : K2 - m];
     Y[idx] = (j & 1) == 0 ? make_float2(0.5f * (z.x + zc.x), 0.5f * (z.y - zc.y))
@@ -466,7 +591,7 @@ __device__ __forceinline__ void pmePlaneForward(const Dev &d, const PmeDev &p, c
   float2 *R = fftBatch(Y, Z, K2h, K1, p.radices[1], tw1, +1);
   float2 *out = p.cgrid + (size_t)i * K1 * K2h;
   for (int idx = t; idx < K1 * K2h; idx += nt) {
-    const int j = idx / K2h, m = idx - j * K2h;
+    const int j = byK2h(idx), m = idx - j * K2h;
     out[idx] = R[m * K1 + j];
   }
 }
@@ -481,13 +606,14 @@ __device__ __forceinline__ void pmeXLines(const Dev &d, const PmeDev &p, int con
   const int chunks = (K2h + XLINES - 1) / XLINES;
   const int j = block / chunks, m0 = (block - j * chunks) * XLINES;
   const int lines = min(XLINES, K2h - m0);
+  const Div byLines(lines);
   const int t = threadIdx.x, nt = blockDim.x;
   float2 *tw = lds, *A = tw + K0, *B = A + XLINES * K0;
   loadTwiddles(tw, p.twiddle[0], K0);
   const size_t stride = (size_t)K1 * K2h;
   float2 *col = p.cgrid + (size_t)j * K2h + m0;
   for (int idx = t; idx < lines * K0; idx += nt) {
-    const int x = idx / lines, l = idx - x * lines;
+    const int x = byLines(idx), l = idx - x * lines;
     A[l * K0 + x] = col[x * stride + l];
   }
   __syncthreads();
@@ -497,7 +623,7 @@ __device__ __forceinline__ void pmeXLines(const Dev &d, const PmeDev &p, int con
     const float *g0 = p.influence + (size_t)j * K2h + m0;
     const double *recip = d.box->recip64;
     for (int idx = t; idx < lines * K0; idx += nt) {
-      const int x = idx / lines, l = idx - x * lines;
+      const int x = byLines(idx), l = idx - x * lines;
       const int m = m0 + l;
       const double weight = (m == 0 || (p.K[2] % 2 == 0 && m == p.K[2] / 2)) ? 1.0 : 2.0;
       const float g = g0[x * stride + l];
@@ -511,7 +637,7 @@ __device__ __forceinline__ void pmeXLines(const Dev &d, const PmeDev &p, int con
     R = fftBatch(R, R == A ? B : A, lines, K0, p.radices[0], tw, -1);
   }
   for (int idx = t; idx < lines * K0; idx += nt) {
-    const int x = idx / lines, l = idx - x * lines;
+    const int x = byLines(idx), l = idx - x * lines;
     col[x * stride + l] = R[l * K0 + x];
   }
   if (convolve && energies) storeReciprocal(d, energy, dscale, block);
@@ -525,11 +651,12 @@ __device__ __forceinline__ void pmeXLines(const Dev &d, const PmeDev &p, int con
 template <bool REAL>
 __device__ __forceinline__ void planeXFold(const PmeDev &p, int i, float2 *A) {
   const int K0 = p.K[0], K1 = p.K[1], K2h = p.K2h, PK = K1 * K2h;
+  const Div byK2h(K2h);
   constexpr int RUN = 16;
   const float *Xr = p.xKernel;
   const float2 *Xc = reinterpret_cast<const float2 *>(p.xKernel);
   for (int c = threadIdx.x; c < PK; c += blockDim.x) {
-    const int j = c / K2h, m = c - j * K2h;
+    const int j = byK2h(c), m = c - j * K2h;
     float re = 0.f, im = 0.f;
     for (int x0 = 0; x0 < K0; x0 += RUN) {
       float2 f[RUN], k[RUN];
@@ -566,8 +693,9 @@ __device__ __forceinline__ void planeXFold(const PmeDev &p, int i, float2 *A) {
 // of read from the x lines' output.
 template <int SCAN = SCAN_PER_THREAD>
 __device__ __forceinline__ void pmePlaneGather(const Dev &d, const PmeDev &p, int i, float2 *lds, int folded = 0) {
-  const int K0 = p.K[0], K1 = p.K[1], K2 = p.K[2], K2h = p.K2h;
+  const int K1 = p.K[1], K2 = p.K[2], K2h = p.K2h;
   const int S = p.planeSpan, P = (K1 + 1) / 2;
+  const Div byK2(K2), byK2h(K2h);
   const int t = threadIdx.x, nt = blockDim.x;
   float2 *tw1 = lds, *tw2 = tw1 + K1;
   float2 *A = tw2 + K2, *B = A + S;
@@ -576,8 +704,9 @@ __device__ __forceinline__ void pmePlaneGather(const Dev &d, const PmeDev &p, in
   // The first scan round's positions are loaded with the plane's spectrum and
   // its list taken before the transforms (the list has LDS of its own), so
   // the positions' load latency overlaps the spectrum's.
+  const bool scanning = p.atoms == PME_ATOMS_SCAN;
   float4 first[SCAN];
-  if (!p.binned) planeScanLoad<SCAN>(d, 0, first);
+  if (scanning) planeScanLoad<SCAN>(d, 0, first);
   loadTwiddles(tw1, p.twiddle[1], K1);
   loadTwiddles(tw2, p.twiddle[2], K2);
   if (folded) {
@@ -588,18 +717,18 @@ __device__ __forceinline__ void pmePlaneGather(const Dev &d, const PmeDev &p, in
   } else {
     const float2 *in = p.cgrid + (size_t)i * K1 * K2h;
     for (int idx = t; idx < K1 * K2h; idx += nt) {
-      const int j = idx / K2h, m = idx - j * K2h;
+      const int j = byK2h(idx), m = idx - j * K2h;
       A[m * K1 + j] = in[idx];
     }
   }
-  if (!p.binned && t == 0) *listCount = 0;
+  if (scanning && t == 0) *listCount = 0;
   __syncthreads();
-  if (!p.binned) planeScanTake<SCAN>(d, p, i, 0, first, list, listCount);
+  if (scanning) planeScanTake<SCAN>(d, p, i, 0, first, list, listCount);
   float2 *Y = fftBatch(A, B, K2h, K1, p.radices[1], tw1, -1);
   float2 *O = (Y == A) ? B : A;
   // Hermitian extension of lines 2p and 2p+1 packed into one complex line.
   for (int idx = t; idx < P * K2; idx += nt) {
-    const int pr = idx / K2, k = idx - pr * K2;
+    const int pr = byK2(idx), k = idx - pr * K2;
     const int j0 = 2 * pr, j1 = 2 * pr + 1;
     float2 a, b = make_float2(0.f, 0.f);
     if (k < K2h) {
@@ -619,14 +748,13 @@ __device__ __forceinline__ void pmePlaneGather(const Dev &d, const PmeDev &p, in
   float2 *Z = fftBatch(O, Y, P, K2, p.radices[2], tw2, -1);
   float *phi = reinterpret_cast<float *>(Z == A ? B : A);
   for (int idx = t; idx < P * K2; idx += nt) {
-    const int pr = idx / K2, k = idx - pr * K2;
+    const int pr = byK2(idx), k = idx - pr * K2;
     phi[2 * pr * K2 + k] = Z[idx].x;
     if (2 * pr + 1 < K1) phi[(2 * pr + 1) * K2 + k] = Z[idx].y;
   }
   __syncthreads();
-  if (p.binned) {
-    // a binned system gathers per atom from the potential grid
-    // (pmeAtomGather)
+  if (!scanning) {
+    // gathered per atom from the potential grid (pmeAtomGather)
     float *out = p.rgrid + (size_t)i * K1 * K2;
     for (int idx = t; idx < K1 * K2; idx += nt) out[idx] = phi[idx];
     return;
@@ -649,9 +777,10 @@ __device__ __forceinline__ void pmePlaneGather(const Dev &d, const PmeDev &p, in
       float w[ORDER], dw[ORDER], wy[ORDER], dwy[ORDER], wz[ORDER], dwz[ORDER];
       bspline5(ox, w, dw);
       float wx = 0.f, dwx = 0.f;
-      for (int q = r; q < ORDER; q += K0) {
-        wx += w[q];
-        dwx += dw[q];
+#pragma unroll
+      for (int q = 0; q < ORDER; ++q) {
+        wx = q == r ? w[q] : wx;
+        dwx = q == r ? dw[q] : dwx;
       }
       gridCoordinate(p, recip, 1, pos, by, oy);
       gridCoordinate(p, recip, 2, pos, bz, oz);

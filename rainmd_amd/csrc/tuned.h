@@ -9,7 +9,7 @@ namespace rmd {
 // batches (kind 1). lanes: direct-space lanes per atom; reach: the widest cell
 // stencil reach the plan may take; searchMode: 0 by cell occupancy, 1 one wave
 // per atom, 2 one wave per cell; skin: nm when the caller asks for the tuned
-// skin (0: the reference's skinFor); pmeBins: 0 by atom count, 1 atom bins,
+// skin (0: the reference's skinFor); pmeBins: 0 by atom count, 1 by cells,
 // 2 every plane scans every atom.
 struct TunedShape {
   int kind, minAtoms, lanes, reach, searchMode;

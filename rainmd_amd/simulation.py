@@ -551,7 +551,7 @@ class GpuSimulation:
         _check(L.load().rmd_set_concurrent_forces(self._h, 1 if enabled else 0), self._h)
 
     def set_pme_pipeline(self, mode):
-        """'auto', 'planes', 'lines', 'planes-scan' (planes without atom bins)
+        """'auto', 'planes', 'lines', 'planes-scan' (planes that scan every atom)
         or 'planes-folded' (planes-scan with the x lines folded into the plane
         gathers on force-only evaluations)."""
         ids = {"auto": 0, "planes": 1, "lines": 2, "planes-scan": 3, "planes-folded": 4}
