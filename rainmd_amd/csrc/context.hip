@@ -288,7 +288,13 @@ void allocateCells(rmd_ctx *c, int cellCount) {
   if (cellCount <= c->d.cellCapacity) return;
   const int capacity = std::max(cellCount, c->d.cellCapacity * 2);
   c->d.cellCount = devAlloc<int>(capacity + 1, c->held);
+  // the cell list in use stays: a volume move may plan more cells than there
+  // is room for without a rebuild, and PME goes by the list as it was built
+  const int *built = c->d.cellStart;
   c->d.cellStart = devAlloc<int>(capacity + 1, c->held);
+  if (built)
+    HIP_CHECK(hipMemcpyAsync(c->d.cellStart, built, sizeof(int) * (c->d.cellCapacity + 1), hipMemcpyDeviceToDevice,
+                             c->stream));
   c->d.cellCursor = devAlloc<int>(capacity + 1, c->held);
   c->d.cellCapacity = capacity;
   invalidateGraphs(c);

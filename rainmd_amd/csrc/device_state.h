@@ -60,7 +60,8 @@ struct Scalars {
   unsigned int spanBits;      // largest atom-to-centroid distance of any molecule seen (float bits)
   long long step;             // the noise counter (completed steps)
   unsigned int cellTicket;    // last-block ticket of the cell assignment
-  unsigned int unused;
+  int builtCells[3];          // the cell counts the cell list was built with (a volume move may plan
+                              // others before the next rebuild)
 };
 
 // A rebuild retires the current list's requirement into requiredMax before

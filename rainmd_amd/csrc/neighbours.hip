@@ -125,6 +125,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) cellsAssignKernel(Dev d) {
   if (t == 0) {
     d.cellStart[total] = carry;
     d.sc->cellTicket = 0u;
+    recordCells(d);
   }
 }
 
@@ -245,6 +246,7 @@ __device__ __forceinline__ void cellsBuildSmall(const Dev &d) {
   const BoxF &box = *d.box;
   const int total = box.cellTotal, n = d.n, t = threadIdx.x;
   for (int c = t; c < total; c += SMALL_THREADS) count[c] = 0;
+  if (t == 0) recordCells(d);
   __syncthreads();
   for (int i = t; i < n; i += SMALL_THREADS) {
     const float4 p = d.pos[i];

@@ -332,7 +332,7 @@ constexpr int SLAB_QUEUE = SLAB_THREADS / 64 * QUEUE_ENTRIES;
 // With more runs than SLAB_RUNS every slot is a candidate.
 __device__ __forceinline__ void slabRuns(const Dev &d, const PmeDev &p, int i, int y0, int rows, SlabRuns &out) {
   const int lane = threadIdx.x;
-  const int cx = d.box->cells[0], cy = d.box->cells[1], cz = d.box->cells[2];
+  const int cx = d.sc->builtCells[0], cy = d.sc->builtCells[1], cz = d.sc->builtCells[2];
   int x0, nx, yFirst, ny;
   supportCells(d, 0, i, 1, p.K[0], x0, nx);
   supportCells(d, 1, y0, rows, p.K[1], yFirst, ny);

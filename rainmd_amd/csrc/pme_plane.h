@@ -340,7 +340,7 @@ __device__ __forceinline__ void planeRanges(const PmeDev &p, int i, int2 range[2
 __device__ __forceinline__ void supportCells(const Dev &d, int axis, int first, int points, int K, int &start,
                                              int &count) {
   const BoxF &b = *d.box;
-  const int cells = b.cells[axis];
+  const int cells = d.sc->builtCells[axis];
   const float moved = 0.5f * (sqrtf(b.rl2) - b.cutoff) + 1e-3f;
   const float r0 = b.recip[axis], r1 = b.recip[3 + axis], r2 = b.recip[6 + axis];
   const float margin = moved * sqrtf(r0 * r0 + r1 * r1 + r2 * r2) + 2e-5f;
@@ -359,7 +359,7 @@ __device__ __forceinline__ void supportCells(const Dev &d, int axis, int first, 
 // The slots a plane's atoms can be in: one run of the cell order (x slowest)
 // or two where it wraps.
 __device__ __forceinline__ void planeSlots(const Dev &d, const PmeDev &p, int i, int2 range[2]) {
-  const int cx = d.box->cells[0], slab = d.box->cells[1] * d.box->cells[2];
+  const int cx = d.sc->builtCells[0], slab = d.sc->builtCells[1] * d.sc->builtCells[2];
   int start, count;
   supportCells(d, 0, i, 1, p.K[0], start, count);
   const int end = start + count;

@@ -30,6 +30,11 @@ __device__ __forceinline__ int cellIndex(float x, float y, float z, const BoxF &
   return (c[0] * cells[1] + c[1]) * cells[2] + c[2];
 }
 
+// The counts a rebuild's cell list is built with, by one thread of it.
+__device__ __forceinline__ void recordCells(const Dev &d) {
+  for (int k = 0; k < 3; ++k) d.sc->builtCells[k] = d.box->cells[k];
+}
+
 // Slot k of the cell order gets atom `atom`: its rebuild-time position with
 // the atom index (for the search), its current position and charge, its type,
 // and the inverse map.
@@ -62,6 +67,7 @@ __device__ void cellsBuildFew(const Dev &d) {
   const BoxF &box = *d.box;
   const int total = box.cellTotal, n = d.n, t = threadIdx.x, lane = t & 63, wave = t >> 6;
   if (t < FEW_MAX_CELLS) cursor[t] = 0;
+  if (t == 0) recordCells(d);
   __syncthreads();
   for (int i = t; i < n; i += THREADS) {
     const float4 p = d.pos[i];

@@ -101,3 +101,30 @@ def test_slab_forces_match_the_oracle(grid):
     sim.release()
     assert rel(gpu["coulomb_reciprocal"], ref["reciprocal"]) < 1e-6
     assert d < FORCE_BAR
+
+
+def test_planes_by_cells_through_volume_moves():
+    """A volume move keeps the cell list and may plan other cell counts before
+    it is rebuilt: the planes go by the counts it was built with. (4.73 nm at
+    a 0.9 nm cutoff: the moves cross from one count per axis to the next.)"""
+    edge, waters, seed = next((e, w, s) for e, w, s in R.replica_workload(32) if w > 3500)
+    system = R.System.solvated(waters, edge, seed, cutoff=0.9)
+    start = R.GpuSimulation(system, temperature=300.0, seed=seed)
+    start.minimise(max_iterations=60, force_tolerance=1000.0)
+    x = start.read_positions().astype(np.float64)
+    start.release()
+    states = {}
+    for mode in ("auto", "planes-scan"):
+        sim = R.GpuSimulation(system, temperature=300.0, seed=seed, pressure=1.0, barostat_interval=5, pme_bins=1)
+        sim.set_pme_pipeline(mode)
+        sim.set_state(x, R.maxwell_boltzmann(system, 300.0, seed))
+        counts = set()
+        for _ in range(12):
+            sim.run(10, 5)
+            counts.add(tuple(sim.diagnostics()["cell_counts"]))
+        d = sim.diagnostics()
+        states[mode] = sim.read_state()
+        print(mode, "cells", counts, "moves", d["barostat_attempts"], "rebuilds", d["rebuilds"], flush=True)
+        sim.release()
+    for name in ("positions", "velocities", "forces"):
+        assert np.array_equal(states["auto"][name], states["planes-scan"][name]), name
