@@ -257,7 +257,10 @@ BoxF boxFor(const rmd_ctx *c, const double *box, const CellPlan &plan) {
   for (int k = 0; k < 3; ++k) b.cells[k] = plan.counts[k];
   b.cellTotal = plan.cellCount;
   b.reach = plan.reach;
-  b.cellSearch = searchByCell(c->searchMode, c->d.n, plan.cellCount) ? 1 : 0;
+  // (a batch fills the chip with its replicas' cells)
+  b.cellSearch = !searchByCell(c->searchMode, c->d.n, plan.cellCount) ? 0
+                 : c->batchMember                                     ? 1
+                                                                      : searchParts(c->d.n, plan.cellCount);
   return b;
 }
 

@@ -37,7 +37,7 @@ struct BoxF {
   int cells[3];
   int cellTotal;
   int reach;  // stencil cells either side (cells are at least rl / reach wide)
-  int cellSearch;  // the list search runs one wave per cell (else one per atom)
+  int cellSearch;  // the list search's waves per cell (0: one wave per atom)
 };
 
 __device__ __forceinline__ long long toFixed(double v) { return static_cast<long long>(__double2ll_rn(v * FORCE_SCALE)); }

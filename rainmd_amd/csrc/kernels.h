@@ -18,6 +18,8 @@ void launchCells(const Dev &d, hipStream_t s);
 // mode: the context's search mode (1 by atom, 2 by cell where the launch
 // covers the cells, 0 by occupancy).
 void launchSearch(const Dev &d, int mode, hipStream_t s);
+// The by-cell search's waves per cell (BoxF::cellSearch).
+int searchParts(int atoms, int cells);
 void launchForceRebuildFlag(const Dev &d, hipStream_t s);
 
 // ---- nonbonded direct space (nonbonded.hip) ----

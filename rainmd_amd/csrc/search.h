@@ -134,9 +134,20 @@ __device__ __forceinline__ void axisStencil(int count, int reach, int &base, int
   }
 }
 
+// A stencil cell's index wrapped into the axis: v lies in [-reach, 2 count)
+// and an axis with a stencil narrower than itself has more than reach cells,
+// so one addition or subtraction wraps it (a remainder by a count known only
+// at run time is some forty instructions).
 __device__ __forceinline__ int wrapCell(int v, int count) {
-  v %= count;
+  v = v >= count ? v - count : v;
   return v < 0 ? v + count : v;
+}
+
+// Stencil row `row` as (row / ny, row % ny), by the reciprocal: exact, (row +
+// 1/2) / ny being at least 1 / 2 ny from an integer.
+__device__ __forceinline__ void stencilRow(int row, int ny, float invNy, int &ix, int &iy) {
+  ix = (int)(((float)row + 0.5f) * invNy);
+  iy = row - ix * ny;
 }
 
 // Whether candidate pj joins atom's list: not itself, within rl (the FP32
@@ -155,6 +166,23 @@ __device__ __forceinline__ bool acceptPair(GlobalPtr<int> excl, const BoxF &box,
   if (accept & (j >= exMin) & (j <= exMax))
     for (int e = exBegin; e < exEnd; ++e)
       if (excl[e] == j) accept = false;
+  return accept;
+}
+
+// acceptPair with the atom and its exclusion partners in atom indices
+// [first, first + span]: one comparison for nearly every candidate.
+template <bool RECT>
+__device__ __forceinline__ bool acceptWithin(GlobalPtr<int> excl, const BoxF &box, float4 pi, float4 pj, int atom,
+                                             int exBegin, int exEnd, int first, unsigned int span) {
+  const int j = __float_as_int(pj.w);
+  float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+  float s0, s1, s2;
+  bool accept = imageR2<RECT>(dx, dy, dz, box, s0, s1, s2) <= box.rl2;
+  if (accept & ((unsigned int)(j - first) <= span)) {
+    accept = j != atom;
+    for (int e = exBegin; e < exEnd; ++e)
+      if (excl[e] == j) accept = false;
+  }
   return accept;
 }
 
@@ -214,6 +242,7 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
     }
   }
   const int ranges = nx * ny * segs;
+  const float invNy = 1.0f / (float)ny;
   int *rb = rangeBegin[wave], *rs = rangeStart[wave];
   // ranges r = lane and lane + 64: their slots and lengths, then an exclusive
   // prefix over all of them
@@ -221,9 +250,11 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
   for (int h = 0; h < 2; ++h) {
     const int r = lane + 64 * h;
     if (r < ranges) {
-      const int row = r / segs, seg = r - row * segs;
-      const int cx = wrapCell(c3[0] + bx + row / ny, cells[0]);
-      const int cy = wrapCell(c3[1] + by + row % ny, cells[1]);
+      const int row = segs == 2 ? r >> 1 : r, seg = r - row * segs;
+      int ix, iy;
+      stencilRow(row, ny, invNy, ix, iy);
+      const int cx = wrapCell(c3[0] + bx + ix, cells[0]);
+      const int cy = wrapCell(c3[1] + by + iy, cells[1]);
       const int rowBase = (cx * cells[1] + cy) * cells[2];
       const int begin = cellStart[rowBase + (seg ? za1 : za0)];
       const int end = cellStart[rowBase + (seg ? zb1 : zb0)];
@@ -289,8 +320,8 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
   return (unsigned int)found;
 }
 
-// One wave per cell. Every atom of a cell has the same stencil, so the wave
-// streams the stencil's candidates as above (the same ranges, in the same
+// One wave per cell, or BoxF::cellSearch of them sharing the cell's atoms.
+// Every atom of a cell has the same stencil, so the wave streams the stencil's candidates as above (the same ranges, in the same
 // order) and tests each candidate against every atom of the cell, up to 64
 // at a time, one per lane, broadcast from its lane in turn. Each atom's
 // accepted candidates are compacted into its own slice in candidate order:
@@ -306,10 +337,13 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
   const GlobalPtr<int> cellStart = globalPtr(d.cellStart);
   const GlobalPtr<int> excl = globalPtr(d.exclPartners);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int cell = block * WAVES + wave;
+  const int parts = d.box->cellSearch, unit = block * WAVES + wave;
+  const int cell = unit / parts, part = unit - cell * parts;
   if (cell >= d.box->cellTotal) return 0u;
   const int cellBegin = cellStart[cell], cellEnd = cellStart[cell + 1];
-  if (cellBegin == cellEnd) return 0u;
+  const int perPart = (cellEnd - cellBegin + parts - 1) / parts;
+  const int ownBegin = cellBegin + part * perPart, ownEnd = min(cellEnd, ownBegin + perPart);
+  if (ownBegin >= ownEnd) return 0u;
   const int c3[3] = {cell / (cells[1] * cells[2]), (cell / cells[2]) % cells[1], cell % cells[2]};
   const int reach = d.box->reach;
   int bx, nx, by, ny, bz, nz;
@@ -363,21 +397,26 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
   }
   // the periodic gap along axis dd between the atoms' box and cell index c:
   // the centres' distance folded into [0, L/2], less both half widths
+  const float widths[3] = {uniformFloat(edge[0] / (float)cells[0]), uniformFloat(edge[1] / (float)cells[1]),
+                           uniformFloat(edge[2] / (float)cells[2])};
   auto gap = [&](int dd, int c) {
-    const float width = edge[dd] / (float)cells[dd];
+    const float width = widths[dd];
     float dist = fabsf((c + 0.5f) * width - centre[dd]);
     dist = fminf(dist, edge[dd] - dist);
     return fmaxf(0.f, dist - half[dd] - 0.5f * width);
   };
   const int ranges = nx * ny * segs;
+  const float invNy = 1.0f / (float)ny;
   int *rb = rangeBegin[wave], *rs = rangeStart[wave];
   int len[2] = {0, 0};
   for (int h = 0; h < 2; ++h) {
     const int r = lane + 64 * h;
     if (r < ranges) {
-      const int row = r / segs, seg = r - row * segs;
-      const int cx = wrapCell(c3[0] + bx + row / ny, cells[0]);
-      const int cy = wrapCell(c3[1] + by + row % ny, cells[1]);
+      const int row = segs == 2 ? r >> 1 : r, seg = r - row * segs;
+      int ix, iy;
+      stencilRow(row, ny, invNy, ix, iy);
+      const int cx = wrapCell(c3[0] + bx + ix, cells[0]);
+      const int cy = wrapCell(c3[1] + by + iy, cells[1]);
       const int rowBase = (cx * cells[1] + cy) * cells[2];
       int zFirst = seg ? za1 : za0, zEnd = seg ? zb1 : zb0;
       if (RECT) {
@@ -420,15 +459,16 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
   const int cap = d.cap;
   constexpr int CAND = 4;
   unsigned int required = 0;
-  for (int first = cellBegin; first < cellEnd; first += 64) {
-    // lane l holds the cell's atom first + l (the last one again past the end)
-    const int atoms = min(64, cellEnd - first);
+  for (int first = ownBegin; first < ownEnd; first += 64) {
+    // lane l holds the wave's atom first + l (the last one again past the end)
+    const int atoms = min(64, ownEnd - first);
     const int own = first + min(lane, atoms - 1);
     const float4 mine = cellPos[own];
     const int myAtom = __float_as_int(mine.w);
     const int myExBegin = d.exclStart[myAtom], myExEnd = d.exclStart[myAtom + 1];
-    const int myExMin = myExBegin < myExEnd ? excl[myExBegin] : 1;
-    const int myExMax = myExBegin < myExEnd ? excl[myExEnd - 1] : 0;
+    // (the partners are sorted)
+    const int myFirst = myExBegin < myExEnd ? min(myAtom, excl[myExBegin]) : myAtom;
+    const int mySpan = (myExBegin < myExEnd ? max(myAtom, excl[myExEnd - 1]) : myAtom) - myFirst;
     if (lane < atoms) d.posRebuild[myAtom] = d.pos[myAtom];
     int myFound = 0;
     int cur = 0;
@@ -445,7 +485,9 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
       }
       float4 p[CAND];
 #pragma unroll
-      for (int u = 0; u < CAND; ++u) p[u] = cellPos[slot[u]];
+      for (int u = 0; u < CAND; ++u) {
+        p[u] = cellPos[slot[u]];
+      }
       for (int i = 0; i < atoms; ++i) {
         const float4 pi = make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.x), i)),
                                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.y), i)),
@@ -453,23 +495,24 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
         const int atom = __builtin_amdgcn_readlane(myAtom, i);
         const int exBegin = __builtin_amdgcn_readlane(myExBegin, i);
         const int exEnd = __builtin_amdgcn_readlane(myExEnd, i);
-        const int exMin = __builtin_amdgcn_readlane(myExMin, i);
-        const int exMax = __builtin_amdgcn_readlane(myExMax, i);
+        const int exFirst = __builtin_amdgcn_readlane(myFirst, i);
+        const unsigned int exSpan = (unsigned int)__builtin_amdgcn_readlane(mySpan, i);
         int found = __builtin_amdgcn_readlane(myFound, i);
         // a lane past the total holds a real atom of the cell: turned down by
         // its position in the stream, not by the pair test
         bool accept[CAND];
 #pragma unroll
         for (int u = 0; u < CAND; ++u)
-          accept[u] = (base + lane + 64 * u < total) &
-                      acceptPair<RECT>(excl, box, pi, p[u], atom, exBegin, exEnd, exMin, exMax);
+          accept[u] = (base + lane + 64 * u < total) & acceptWithin<RECT>(excl, box, pi, p[u], atom, exBegin, exEnd, exFirst, exSpan);
         const GlobalOut<int> out = globalOut(d.nbrList + (size_t)(first + i) * cap);
 #pragma unroll
         for (int u = 0; u < CAND; ++u) {
           const unsigned long long mask = __ballot(accept[u]);
           if (accept[u]) {
-            const int where = found + __popcll(mask & ((1ull << lane) - 1ull));
-            if (where < cap) out[where] = slot[u];
+            // found + the accepted lanes below this one
+            const unsigned int where = __builtin_amdgcn_mbcnt_hi(
+                (unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, (unsigned int)found));
+            if (where < (unsigned int)cap) out[where] = slot[u];
           }
           found += __popcll(mask);
         }
