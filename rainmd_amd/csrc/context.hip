@@ -1138,6 +1138,7 @@ void create(rmd_ctx *c, const System &sys, const rmd_options &o, const Streams *
   d.box = c->boxDev;
   d.type = devAlloc<int>(d.nPad, c->held);
   d.types = t.typeCount;
+  d.typeInList = typesInList(d.types, n) ? 1 : 0;
   {
     std::vector<float2> lj(t.ljA.size());
     for (size_t k = 0; k < lj.size(); ++k) lj[k] = make_float2((float)t.ljA[k], (float)t.ljB[k]);
@@ -2040,7 +2041,10 @@ int rmd_read_neighbours(rmd_ctx *c, int32_t *counts, int32_t *lists) {
       HIP_CHECK(hipMemcpy(rows.data(), c->d.nbrList, rows.size() * sizeof(int), hipMemcpyDeviceToHost));
       for (int r = 0; r < n; ++r) {
         int32_t *dst = lists + (size_t)atomOf[r] * cap;
-        for (int k = 0; k < cap; ++k) dst[k] = k < rowCount[r] ? atomOf[rows[(size_t)r * cap + k]] : 0;
+        for (int k = 0; k < cap; ++k) {
+          const int entry = k < rowCount[r] ? rows[(size_t)r * cap + k] : 0;
+          dst[k] = k < rowCount[r] ? atomOf[c->d.typeInList ? listSlot(entry) : entry] : 0;
+        }
       }
     }
   });
@@ -2368,6 +2372,7 @@ struct rmd_batch {
   double alpha = 0;
   int lanes = 16;  // direct-space lanes per atom of every member
   int maxTypes = 0;  // the largest LJ type count of the members
+  int typeInList = 1;  // every member's list carries its neighbours' types
   int allRect = 1;   // every member's box is rectangular
   int rational = 1;  // the direct-space Coulomb force from the rational fit for every member
   bool concurrent = true, useGraphs = true;
@@ -2555,7 +2560,7 @@ void enqueueBatchForces(rmd_batch *b, int energies, int terms = RMD_TERM_ALL) {
                      st.stream);
   if (terms & RMD_TERM_DIRECT)
     launchNonbondedBatch(b->dViews, b->tables[BK_NONBONDED], b->lanes, (float)b->alpha, b->rational, energies,
-                         b->maxTypes, b->allRect, st.stream);
+                         b->maxTypes, b->typeInList, b->allRect, st.stream);
   if (fork) {
     for (int k = 0; k < 2; ++k) {
       HIP_CHECK(hipEventRecord(st.join[k], st.side[k]));
@@ -2971,6 +2976,7 @@ void createBatch(rmd_batch *b, const rmd_system *const *systems, int count, cons
       throw Error(RMD_E_INVALID, replicaLabel(r) + "every replica of a batch needs the same Ewald alpha (the same "
                                                    "cutoff and tolerance)");
     b->maxTypes = std::max(b->maxTypes, c->d.types);
+    b->typeInList = b->typeInList && c->d.typeInList;
     b->allRect = b->allRect && c->d.rect;
     b->rational = b->rational && ewaldRationalFits(c->pme.alpha, c->sys.cutoff);
     b->ldsForward = std::max(b->ldsForward, pmePlaneForwardLds(c->p));
@@ -2979,6 +2985,8 @@ void createBatch(rmd_batch *b, const rmd_system *const *systems, int count, cons
     b->ldsOpen = std::max(b->ldsOpen, c->ip.clusterLdsBytes);
     b->starMax = std::max(b->starMax, c->ip.starMax);
   }
+  // one form of the list for every member, stepped together or alone
+  for (rmd_ctx *c : b->reps) c->d.typeInList = b->typeInList;
   pmeBatchLdsLimits(b->ldsForward, b->ldsXlines, b->ldsGather);
   for (int k = 0; k < BK_COUNT; ++k) b->tables[k] = buildTasks(b, k);
   // The list search: at most 1024 workgroups per XCD (enough to fill the chip
@@ -3172,14 +3180,14 @@ int rmd_batch_profile_nonbonded(rmd_batch *b, int32_t reps, double *avg_ms) {
     hipStream_t s = b->streams.stream;
     uploadViews(b);
     launchNonbondedBatch(b->dViews, b->tables[BK_NONBONDED], b->lanes, (float)b->alpha, b->rational, 0, b->maxTypes,
-                         b->allRect, s);
+                         b->typeInList, b->allRect, s);
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
     HIP_CHECK(hipEventRecord(e0, s));
     for (int k = 0; k < reps; ++k)
       launchNonbondedBatch(b->dViews, b->tables[BK_NONBONDED], b->lanes, (float)b->alpha, b->rational, 0, b->maxTypes,
-                         b->allRect, s);
+                         b->typeInList, b->allRect, s);
     HIP_CHECK(hipEventRecord(e1, s));
     HIP_CHECK(hipEventSynchronize(e1));
     float ms = 0;

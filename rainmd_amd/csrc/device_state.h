@@ -98,7 +98,8 @@ struct Dev {
   const BoxF *box;  // device-resident geometry (see BoxF)
   // cells (arrays sized for cellCapacity cells)
   int *cellOfAtom, *cellCount, *cellStart, *cellCursor, *cellAtoms;
-  float4 *cellPos;  // positions in cell order at the last rebuild, the atom index in .w (int bits)
+  float4 *cellPos;  // positions in cell order at the last rebuild, the atom index in .w (int bits; with
+                    // typeInList its type above it, as in a list entry)
   int cellCapacity;
   // The current positions (.w the charge) and types in cell order ("slots":
   // slot k holds atom cellAtoms[k]); the integrator keeps slotPos current
@@ -109,6 +110,7 @@ struct Dev {
   // neighbours: full list, `cap` slots per atom
   int *nbrCount, *nbrList;
   int cap;
+  int typeInList;  // entries carry the neighbour's type above its slot (listEntry)
   int *exclStart, *exclPartners;
   // bonded terms (f32 parameters)
   int nBond, nAngle, nTorsion, nException, nRestraint;

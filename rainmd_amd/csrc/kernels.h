@@ -23,6 +23,7 @@ int searchParts(int atoms, int cells);
 void launchForceRebuildFlag(const Dev &d, hipStream_t s);
 
 // ---- nonbonded direct space (nonbonded.hip) ----
+bool typesInList(int types, int atoms);
 // lanes: lanes per atom (1, 2, 4, ..., 64). energies != 0 fills the
 // E_LJ_DIRECT / E_COUL_DIRECT slot rows and returns the slot count used.
 // rational: the screened Coulomb force from the rational fit (alpha * cutoff
@@ -294,7 +295,7 @@ void launchRebuildBatch(const BatchView *v, const TaskTable &replicaTable, int r
 int searchQueueInts(int replicas);
 // lanes: lanes per atom (8, 16, 32 or 64), the table's grid at that count.
 void launchNonbondedBatch(const BatchView *v, const TaskTable &t, int lanes, float alpha, int rational, int energies,
-                          int types, int rect, hipStream_t s);
+                          int types, int typeInList, int rect, hipStream_t s);
 void launchBondedBatch(const BatchView *v, const TaskTable &t, double alpha, int terms, int energies, hipStream_t s);
 void launchPmeBatch(const BatchView *v, const TaskTable &planes, const TaskTable &xlines, const TaskTable &replicas,
                     const TaskTable &atoms256, int energies, size_t forwardLds, size_t xlinesLds, size_t gatherLds,

@@ -26,8 +26,11 @@ namespace rmd {
 // the system; larger ones are read from global memory.
 constexpr int LDS_TYPES = 90;
 
-inline bool tableInLds(int types) { return types <= LDS_TYPES; }
-inline size_t tableLdsBytes(int types) { return tableInLds(types) ? (size_t)types * types * sizeof(float2) : 0; }
+// Whether a system keeps its type table in LDS, and with it its neighbours'
+// types in the list (Dev::typeInList).
+bool typesInList(int types, int atoms) { return types <= LDS_TYPES && atoms <= (1 << LIST_SLOT_BITS); }
+inline size_t tableLdsBytes(int types) { return (size_t)types * types * sizeof(float2); }
+inline size_t tableLdsBytes(const Dev &d) { return d.typeInList ? tableLdsBytes(d.types) : 0; }
 
 // G(w) = (erf(z) - 2 z / sqrt(pi) exp(-w)) / z^3 with w = z^2 = (alpha r)^2,
 // as P(w) / Q(w) of degree 5 (a relative-error fit on [0, 12] made for this
@@ -171,8 +174,9 @@ __device__ __forceinline__ void nonbonded(const Dev &d, float alpha, int block, 
       int t[UNROLL];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-        p[u] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(posBuffer, j[u] * 16, 0, 0));
-        t[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(typeBuffer, j[u] * 4, 0, 0);
+        const int slot = LDS_TABLE ? listSlot(j[u]) : j[u];
+        p[u] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(posBuffer, slot * 16, 0, 0));
+        t[u] = LDS_TABLE ? listType(j[u]) : (int)__builtin_amdgcn_raw_buffer_load_b32(typeBuffer, slot * 4, 0, 0);
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
@@ -378,8 +382,8 @@ static void dispatch(const Variant &k, bool batch, const Dev *d, const BatchView
 int launchNonbonded(const Dev &d, float alpha, int rational, int lanes, int energies, hipStream_t s) {
   const long long threads = (long long)d.n * lanes;
   const int blocks = (int)((threads + 255) / 256);
-  const Variant k{energies != 0, tableInLds(d.types), d.rect != 0, rational != 0};
-  dispatch(k, false, &d, nullptr, nullptr, alpha, lanes, blocks, tableLdsBytes(d.types), s);
+  const Variant k{energies != 0, d.typeInList != 0, d.rect != 0, rational != 0};
+  dispatch(k, false, &d, nullptr, nullptr, alpha, lanes, blocks, tableLdsBytes(d), s);
   return blocks;
 }
 
@@ -390,14 +394,14 @@ int launchNonbonded(const Dev &d, float alpha, int rational, int lanes, int ener
 // plane pipeline scanning every atom and at most 64 KB of LDS per workgroup.
 bool forcesJoin(const Dev &d, const PmeDev &p, int lanes) {
   constexpr long long ONE_PASS = 256LL * 4 * 4 * 64;  // threads
-  return (lanes == 16 || lanes == 32 || lanes == 64) && (long long)d.n * lanes <= ONE_PASS && tableInLds(d.types) &&
-         p.planes && p.atoms == PME_ATOMS_SCAN && std::max(tableLdsBytes(d.types), pmePlaneForwardLds(p)) <= 65536;
+  return (lanes == 16 || lanes == 32 || lanes == 64) && (long long)d.n * lanes <= ONE_PASS && d.typeInList &&
+         p.planes && p.atoms == PME_ATOMS_SCAN && std::max(tableLdsBytes(d), pmePlaneForwardLds(p)) <= 65536;
 }
 
 void launchForcesJoined(const Dev &d, const PmeDev &p, float alpha, int rational, int lanes, int energies,
                         double alphaD, int terms, hipStream_t s, int *pairSlots, int *bondedSlots, int search) {
   const Variant k{energies != 0, true, d.rect != 0, rational != 0};
-  const size_t lds = std::max(tableLdsBytes(d.types), pmePlaneForwardLds(p));
+  const size_t lds = std::max(tableLdsBytes(d), pmePlaneForwardLds(p));
   dispatch(k, false, &d, nullptr, nullptr, alpha, lanes, 0, lds, s, JoinedPart{&p, alphaD, terms, search});
   // energy slots as the 256-thread kernels number them
   *pairSlots = (int)(((long long)d.n * lanes + 255) / 256);
@@ -405,11 +409,12 @@ void launchForcesJoined(const Dev &d, const PmeDev &p, float alpha, int rational
 }
 
 // `types` is the largest type count of the batch's replicas: every workgroup
-// gets LDS for that table. `rect`: every replica's box is rectangular.
+// gets LDS for that table, where every replica's list carries the types
+// (`typeInList`). `rect`: every replica's box is rectangular.
 void launchNonbondedBatch(const BatchView *v, const TaskTable &t, int lanes, float alpha, int rational, int energies,
-                          int types, int rect, hipStream_t s) {
-  const Variant k{energies != 0, tableInLds(types), rect != 0, rational != 0};
-  dispatch(k, true, nullptr, v, &t, alpha, lanes, 0, tableLdsBytes(types), s);
+                          int types, int typeInList, int rect, hipStream_t s) {
+  const Variant k{energies != 0, typeInList != 0, rect != 0, rational != 0};
+  dispatch(k, true, nullptr, v, &t, alpha, lanes, 0, typeInList ? tableLdsBytes(types) : 0, s);
 }
 
 }  // namespace rmd

@@ -36,11 +36,12 @@ __device__ __forceinline__ void recordCells(const Dev &d) {
 }
 
 // Slot k of the cell order gets atom `atom`: its rebuild-time position with
-// the atom index (for the search), its current position and charge, its type,
+// the atom index, under its type where the list carries types (for the
+// search), its current position and charge, its type,
 // and the inverse map.
 __device__ __forceinline__ void writeSlotLoaded(const Dev &d, int k, int atom, float4 p, int type) {
   d.cellAtoms[k] = atom;
-  d.cellPos[k] = make_float4(p.x, p.y, p.z, __int_as_float(atom));
+  d.cellPos[k] = make_float4(p.x, p.y, p.z, __int_as_float(d.typeInList ? listEntry(atom, type) : atom));
   d.slotPos[k] = p;
   d.slotType[k] = type;
   d.slotOf[atom] = k;
@@ -154,11 +155,11 @@ __device__ __forceinline__ void stencilRow(int row, int ny, float invNy, int &ix
 // minimum image of the kernels), not excluded. Exclusions are checked only
 // for candidates inside the range of the atom's (sorted) exclusion partners.
 template <bool RECT>
-__device__ __forceinline__ bool acceptPair(GlobalPtr<int> excl, const BoxF &box, float4 pi, float4 pj, int atom,
-                                           int exBegin, int exEnd, int exMin, int exMax) {
+__device__ __forceinline__ bool acceptPair(GlobalPtr<int> excl, const BoxF &box, float4 pi, float4 pj, int indexBits,
+                                           int atom, int exBegin, int exEnd, int exMin, int exMax) {
   // the distance test first and without a branch, so the candidate's loads
   // are used whole where they are issued
-  const int j = __float_as_int(pj.w);
+  const int j = __float_as_int(pj.w) & indexBits;
   float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
   float s0, s1, s2;
   const float r2 = imageR2<RECT>(dx, dy, dz, box, s0, s1, s2);
@@ -172,9 +173,9 @@ __device__ __forceinline__ bool acceptPair(GlobalPtr<int> excl, const BoxF &box,
 // acceptPair with the atom and its exclusion partners in atom indices
 // [first, first + span]: one comparison for nearly every candidate.
 template <bool RECT>
-__device__ __forceinline__ bool acceptWithin(GlobalPtr<int> excl, const BoxF &box, float4 pi, float4 pj, int atom,
-                                             int exBegin, int exEnd, int first, unsigned int span) {
-  const int j = __float_as_int(pj.w);
+__device__ __forceinline__ bool acceptWithin(GlobalPtr<int> excl, const BoxF &box, float4 pi, float4 pj,
+                                             int indexBits, int atom, int exBegin, int exEnd, int first, unsigned int span) {
+  const int j = __float_as_int(pj.w) & indexBits;
   float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
   float s0, s1, s2;
   bool accept = imageR2<RECT>(dx, dy, dz, box, s0, s1, s2) <= box.rl2;
@@ -204,6 +205,7 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
   const int cells[3] = {d.box->cells[0], d.box->cells[1], d.box->cells[2]};
   const GlobalPtr<float4> cellPos = globalPtr(d.cellPos);
   const GlobalPtr<int> cellStart = globalPtr(d.cellStart);
+  const int indexBits = d.typeInList ? listSlot(-1) : -1;  // of a cellPos .w: the atom index, below its type
   const GlobalPtr<int> excl = globalPtr(d.exclPartners);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int row = (block * blockDim.x + threadIdx.x) >> 6;  // a slot
@@ -279,7 +281,7 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
   int found = 0;
   const GlobalOut<int> out = globalOut(d.nbrList + (size_t)row * d.cap);
   const int cap = d.cap;
-  auto emit = [&](bool accept, int j) {  // j: the candidate's slot
+  auto emit = [&](bool accept, int j) {  // j: the candidate's entry
     const unsigned long long mask = __ballot(accept);
     if (accept) {
       const int where = found + __popcll(mask & ((1ull << lane) - 1ull));
@@ -310,10 +312,10 @@ __device__ __forceinline__ unsigned int neighbours(const Dev &d, int block) {
     // completion counter)
     bool accept[CAND];
 #pragma unroll
-    for (int u = 0; u < CAND; ++u) accept[u] = acceptPair<RECT>(excl, box, pi, p[u], atom, exBegin, exEnd, exMin, exMax);
+    for (int u = 0; u < CAND; ++u) accept[u] = acceptPair<RECT>(excl, box, pi, p[u], indexBits, atom, exBegin, exEnd, exMin, exMax);
 #pragma unroll
     for (int u = 0; u < CAND; ++u)
-      if (base + 64 * u < total) emit(accept[u], slot[u]);
+      if (base + 64 * u < total) emit(accept[u], slot[u] | (__float_as_int(p[u].w) & ~indexBits));
   }
   __builtin_amdgcn_wave_barrier();
   if (lane == 0) d.nbrCount[row] = found < cap ? found : cap;
@@ -335,6 +337,7 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
   const int cells[3] = {d.box->cells[0], d.box->cells[1], d.box->cells[2]};
   const GlobalPtr<float4> cellPos = globalPtr(d.cellPos);
   const GlobalPtr<int> cellStart = globalPtr(d.cellStart);
+  const int indexBits = d.typeInList ? listSlot(-1) : -1;  // of a cellPos .w: the atom index, below its type
   const GlobalPtr<int> excl = globalPtr(d.exclPartners);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int parts = d.box->cellSearch, unit = block * WAVES + wave;
@@ -464,7 +467,7 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
     const int atoms = min(64, ownEnd - first);
     const int own = first + min(lane, atoms - 1);
     const float4 mine = cellPos[own];
-    const int myAtom = __float_as_int(mine.w);
+    const int myAtom = __float_as_int(mine.w) & indexBits;
     const int myExBegin = d.exclStart[myAtom], myExEnd = d.exclStart[myAtom + 1];
     // (the partners are sorted)
     const int myFirst = myExBegin < myExEnd ? min(myAtom, excl[myExBegin]) : myAtom;
@@ -503,7 +506,7 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
         bool accept[CAND];
 #pragma unroll
         for (int u = 0; u < CAND; ++u)
-          accept[u] = (base + lane + 64 * u < total) & acceptWithin<RECT>(excl, box, pi, p[u], atom, exBegin, exEnd, exFirst, exSpan);
+          accept[u] = (base + lane + 64 * u < total) & acceptWithin<RECT>(excl, box, pi, p[u], indexBits, atom, exBegin, exEnd, exFirst, exSpan);
         const GlobalOut<int> out = globalOut(d.nbrList + (size_t)(first + i) * cap);
 #pragma unroll
         for (int u = 0; u < CAND; ++u) {
@@ -512,7 +515,7 @@ __device__ __forceinline__ unsigned int neighboursByCell(const Dev &d, int block
             // found + the accepted lanes below this one
             const unsigned int where = __builtin_amdgcn_mbcnt_hi(
                 (unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, (unsigned int)found));
-            if (where < (unsigned int)cap) out[where] = slot[u];
+            if (where < (unsigned int)cap) out[where] = slot[u] | (__float_as_int(p[u].w) & ~indexBits);
           }
           found += __popcll(mask);
         }
