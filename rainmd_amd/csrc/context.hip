@@ -115,6 +115,13 @@ struct ReadBack {
   unsigned int rebuildsBefore;
 };
 
+// What an evaluation hands back to the host, in pinned memory.
+struct EvaluationBack {
+  Scalars sc;
+  double terms[E_TERM_COUNT];
+  unsigned int maxForceBits;
+};
+
 struct rmd_ctx {
   System sys;
   // A member of a replica batch: the batch owns it (rmd_destroy leaves it
@@ -176,8 +183,8 @@ struct rmd_ctx {
   double *dTermsTrial = nullptr;
   // what a block hands back, gathered on the device for one copy
   ReadBack *readBack = nullptr;
-  // Pinned memory the read-backs of positions, velocities and forces are
-  // packed into by the device (readArrays).
+  // Pinned memory the device writes read-backs to: an evaluation's
+  // (EvaluationBack), then positions, velocities and forces (readArrays).
   void *readStage = nullptr;
   int64_t blockEndStep = -1;
   unsigned int *dMaxForce = nullptr;
@@ -549,9 +556,13 @@ __global__ void setStepKernel(Scalars *sc, long long step) { sc->step = step; }
 // and joined before anything that reads the forces. Forces are int64 atomics and every energy has its own slot row,
 // so the results do not depend on the overlap.
 // `molecular`: energies with the molecular scaling term; `cellsBuilt`: the
-// step's integrator has built the cell list.
+// step's integrator has built the cell list; `rebuilding`: the list is rebuilt
+// for certain, so its search takes a launch of its own, every row's wave at
+// once, where the joined launch, which a step runs far more often without a
+// rebuild, goes through its rows in passes (2854 atoms: 66.6 us joined, 33.5
+// and 20.2 us apart).
 void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT], bool molecular = true,
-                   bool cellsBuilt = false) {
+                   bool cellsBuilt = false, bool rebuilding = false) {
   Dev &d = c->d;
   for (int k = 0; k < E_TERM_COUNT; ++k) slots[k] = 0;
   const int bondedMask = RMD_TERM_BONDED | RMD_TERM_EXCEPTIONS | RMD_TERM_RESTRAINT;
@@ -564,7 +575,7 @@ void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT],
                       (terms & bondedMask) && forcesJoin(d, c->p, c->lanes);
   if (joined) {
     // the one-wave-per-atom search runs in the joined launch
-    const bool searchJoined = !searchByCell(c->searchMode, d.n, c->plan.cellCount);
+    const bool searchJoined = !rebuilding && !searchByCell(c->searchMode, d.n, c->plan.cellCount);
     if (!cellsBuilt) launchCells(d, c->stream);
     if (!searchJoined) launchSearch(d, c->searchMode, c->stream);
     int pair = 0, bonded = 0;
@@ -615,32 +626,61 @@ void enqueueForces(rmd_ctx *c, int terms, int energies, int slots[E_TERM_COUNT],
                              "or too small for this cutoff");
 }
 
-void checkScalars(rmd_ctx *c, Scalars &h) {
-  HIP_CHECK(hipMemcpyAsync(&h, c->d.sc, sizeof h, hipMemcpyDeviceToHost, c->stream));
-  HIP_CHECK(hipStreamSynchronize(c->stream));
-  if (h.cellOverflow) cellOverflowError();
+// The context's pinned memory, made at its first use for everything read
+// through it (allocating some takes 0.3 ms and more): an evaluation's results,
+// then the widest read of the state (12 bytes a number: three floats, or the
+// doubles alone).
+constexpr size_t STAGE_ARRAYS = (sizeof(EvaluationBack) + 255) / 256 * 256;
+char *readStage(rmd_ctx *c) {
+  if (!c->readStage)
+    HIP_CHECK(hipHostMalloc(&c->readStage, STAGE_ARRAYS + 9 * sizeof(float) * (size_t)c->d.n, hipHostMallocDefault));
+  return static_cast<char *>(c->readStage);
+}
+
+// An evaluation's results straight to pinned memory, so that its one wait is
+// all the host does (a copy to pageable memory each for the Scalars, the
+// energies and the largest force took about 10 us apiece). Leaves the largest
+// force cleared for the next evaluation.
+__global__ void gatherEvaluationKernel(const Scalars *sc, const double *terms, unsigned int *maxForce,
+                                       EvaluationBack *out) {
+  const int t = threadIdx.x;
+  if (t == 0) out->sc = *sc;
+  if (terms && t < E_TERM_COUNT) out->terms[t] = terms[t];
+  if (maxForce && t == 0) {
+    out->maxForceBits = *maxForce;
+    *maxForce = 0u;
+  }
 }
 
 // One evaluation at the current positions. force_rebuild mirrors the
 // reference's #evaluatePotential, which always rebuilds.
-void evaluate(rmd_ctx *c, int terms, bool forceRebuild, double terms_out[E_TERM_COUNT]) {
+// `molecular`: the energies with the molecular scaling term; `maxForce`: the
+// largest force on any atom.
+void evaluate(rmd_ctx *c, int terms, bool forceRebuild, double terms_out[E_TERM_COUNT], bool molecular = true,
+              double *maxForce = nullptr) {
   for (int attempt = 0; attempt < 4; ++attempt) {
     beginEvaluationKernel<<<(c->d.nPad + 255) / 256, 256, 0, c->stream>>>(c->d, c->ip.dispHalf,
                                                                           forceRebuild ? 1 : 0, 0);
     int slots[E_TERM_COUNT];
-    enqueueForces(c, terms, terms_out ? 1 : 0, slots);
+    enqueueForces(c, terms, terms_out ? 1 : 0, slots, molecular, false, forceRebuild);
+    // reduced and handed over before the one wait below (discarded if the
+    // list overflowed and the evaluation runs again)
     if (terms_out) {
-      // reduced and copied before the one wait below (discarded if the list
-      // overflowed and the evaluation runs again)
       SlotCounts counts;
       std::memcpy(counts.c, slots, sizeof slots);
       launchReduceEnergies(c->d, counts, c->dTerms, c->stream);
-      HIP_CHECK(hipMemcpyAsync(terms_out, c->dTerms, sizeof(double) * E_TERM_COUNT, hipMemcpyDeviceToHost,
-                               c->stream));
     }
+    if (maxForce) launchMaxForce(c->d, c->dMaxForce, c->stream);
+    static_assert(E_TERM_COUNT <= 64, "one thread per energy term");
+    EvaluationBack &back = *reinterpret_cast<EvaluationBack *>(readStage(c));
+    gatherEvaluationKernel<<<1, 64, 0, c->stream>>>(c->d.sc, terms_out ? c->dTerms : nullptr,
+                                                    maxForce ? c->dMaxForce : nullptr, &back);
     HIP_CHECK(hipGetLastError());
-    Scalars h;
-    checkScalars(c, h);
+    HIP_CHECK(hipStreamSynchronize(c->stream));
+    const Scalars &h = back.sc;
+    if (h.cellOverflow) cellOverflowError();
+    if (terms_out) std::memcpy(terms_out, back.terms, sizeof back.terms);
+    if (maxForce) *maxForce = (double)__builtin_bit_cast(float, back.maxForceBits);
     c->rebuildCount = h.rebuilds;
     const unsigned int need = requirementSince(h);
     c->worstRequired = std::max(c->worstRequired, need);
@@ -763,9 +803,10 @@ void trainScreen(ScreenState &sc, int device) {
 
 void screenTrain(rmd_ctx *c) { trainScreen(c->screen, c->device); }
 
-double evaluatePotential(rmd_ctx *c) {
+// The potential and the largest force with a fresh list (the minimiser's).
+double evaluatePotential(rmd_ctx *c, double *maxForce) {
   double t[E_TERM_COUNT];
-  evaluate(c, RMD_TERM_ALL, true, t);
+  evaluate(c, RMD_TERM_ALL, true, t, false, maxForce);
   return potentialFromTerms(c, t);
 }
 
@@ -989,14 +1030,11 @@ __global__ void __launch_bounds__(256) packStateKernel(Dev d, float *pos, float 
   }
 }
 
-// Reads what is not null into the caller's arrays. The stage is made at the
-// first read, for the widest one (12 bytes a number: three floats, or the
-// doubles alone): allocating pinned memory takes 0.3 ms and more.
+// Reads what is not null into the caller's arrays.
 void readArrays(rmd_ctx *c, float *pos, float *vel, float *force, double *force64) {
   const size_t n3 = 3 * (size_t)c->d.n;
   if (!pos && !vel && !force && !force64) return;
-  if (!c->readStage) HIP_CHECK(hipHostMalloc(&c->readStage, n3 * 3 * sizeof(float), hipHostMallocDefault));
-  char *at = static_cast<char *>(c->readStage);
+  char *at = readStage(c) + STAGE_ARRAYS;
   auto take = [&](size_t bytes) {
     char *p = at;
     at += bytes;
@@ -1910,56 +1948,45 @@ int rmd_minimise(rmd_ctx *c, const rmd_min_options *options, rmd_min_result *out
     rmd_min_options_default(&o);
     if (options) o = *options;
     double maxStep = o.max_step;
-    const size_t np = c->d.nPad;
-    auto maxForce = [&]() {
-      HIP_CHECK(hipMemsetAsync(c->dMaxForce, 0, sizeof(unsigned int), c->stream));
-      launchMaxForce(c->d, c->dMaxForce, c->stream);
-      unsigned int bits = 0;
-      HIP_CHECK(hipMemcpyAsync(&bits, c->dMaxForce, sizeof bits, hipMemcpyDeviceToHost, c->stream));
-      HIP_CHECK(hipStreamSynchronize(c->stream));
-      return (double)__builtin_bit_cast(float, bits);
-    };
-    double potential = evaluatePotential(c);
+    // Every trial moves from the saved base point along its forces (the first
+    // saves it), and a trial's largest force comes back with its potential,
+    // so an attempt is one chain of launches and one wait.
+    double worst = 0;
+    double potential = evaluatePotential(c, &worst);
     int iterations = 0, rejected = 0;
     bool stalled = false;
-    double worst = 0;
     for (int it = 0; it < o.max_iterations; ++it) {
       iterations = it + 1;
-      worst = maxForce();
       if (worst <= o.force_tolerance) break;
-      HIP_CHECK(hipMemcpyAsync(c->posSaved, c->d.pos, np * sizeof(float4), hipMemcpyDeviceToDevice, c->stream));
-      HIP_CHECK(hipMemcpyAsync(c->forceSaved, c->d.force, 3 * np * sizeof(long long), hipMemcpyDeviceToDevice, c->stream));
       bool accepted = false;
       for (int attempt = 0; attempt < 14; ++attempt) {
-        launchDisplace(c->d, (float)(maxStep / std::max(worst, 1e-6)), (float)o.max_displacement, c->stream);
+        launchDisplace(c->d, c->posSaved, c->forceSaved, attempt > 0, (float)(maxStep / std::max(worst, 1e-6)),
+                       (float)o.max_displacement, c->stream);
         launchConstrainPositions(c->d, c->posSaved, c->ip, c->stream);
-        const double trial = evaluatePotential(c);
+        double trialWorst = 0;
+        const double trial = evaluatePotential(c, &trialWorst);
         if (trial < potential) {
           potential = trial;
+          worst = trialWorst;
           maxStep *= 1.3;
           accepted = true;
           break;
         }
         rejected += 1;
-        // Back to the pre-move positions AND forces: the next, smaller step
-        // goes along the gradient at the base point.
-        HIP_CHECK(hipMemcpyAsync(c->d.pos, c->posSaved, np * sizeof(float4), hipMemcpyDeviceToDevice, c->stream));
-        HIP_CHECK(hipMemcpyAsync(c->d.force, c->forceSaved, 3 * np * sizeof(long long), hipMemcpyDeviceToDevice, c->stream));
         maxStep *= 0.5;
         if (maxStep < 1e-9) break;
       }
       if (!accepted) {
+        // Back to the pre-move positions AND forces.
+        launchSnapshot(c->d, SnapshotBuffers{c->posSaved, nullptr, nullptr, c->forceSaved, nullptr, nullptr},
+                       SNAP_RESTORE, c->stream);
         stalled = true;
         break;
       }
     }
-    worst = maxForce();
     // Velocities are zeroed, as the reference does after minimising.
-    std::vector<float4> v(np);
-    HIP_CHECK(hipMemcpyAsync(v.data(), c->d.vel, np * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
-    for (auto &x : v) x.x = x.y = x.z = 0.f;
-    HIP_CHECK(hipMemcpyAsync(c->d.vel, v.data(), np * sizeof(float4), hipMemcpyHostToDevice, c->stream));
+    launchZeroVelocities(c->d, c->stream);
+    HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(c->stream));
     c->initialised = true;
     if (out) {

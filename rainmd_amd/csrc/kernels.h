@@ -180,7 +180,11 @@ int launchMolecularTerm(const Dev &d, const int *molStart, const int *molAtoms, 
 // Minimiser helpers.
 void launchMaxForce(const Dev &d, unsigned int *out, hipStream_t s);
 void launchNoise(int n, unsigned int seed, unsigned int step, float *uniforms, float *normals, hipStream_t s);
-void launchDisplace(const Dev &d, float scale, float cap, hipStream_t s);
+// x = base + clamp(scale * F_base, cap) per atom: the base point is the
+// current state, saved first, or with `again` the saved one.
+void launchDisplace(const Dev &d, float4 *posSaved, long long *forceSaved, bool again, float scale, float cap,
+                    hipStream_t s);
+void launchZeroVelocities(const Dev &d, hipStream_t s);
 void launchConstrainPositions(const Dev &d, const float4 *reference, const IntegratorParams &ip, hipStream_t s);
 
 // ---- replica batches ----------------------------------------------------------
