@@ -546,15 +546,16 @@ __global__ void __launch_bounds__(256) beginEvaluationKernel(Dev d, double dispH
 __global__ void setForceRebuildKernel(Scalars *sc) { sc->forceRebuild = 1u; }
 __global__ void setStepKernel(Scalars *sc, long long step) { sc->step = step; }
 
-// One force evaluation. A small system runs its direct space, bonded terms
-// and PME forward planes as one launch after the list rebuild, then the rest
-// of PME, all on the context's stream: a captured step runs forked branches
-// one after another, so separate launches cost the sum of their durations,
-// where one launch overlaps them. Otherwise the cell list comes first; PME,
-// the longest branch, stays on the context's stream, and the list search with
-// the direct space, and the bonded terms, run on side streams forked after it
-// and joined before anything that reads the forces. Forces are int64 atomics and every energy has its own slot row,
-// so the results do not depend on the overlap.
+// One force evaluation. A system whose direct space fits the chip in one pass
+// runs it, its bonded terms and its PME forward planes as one launch after the
+// list rebuild, then the rest of PME, all on the context's stream: a captured
+// step runs forked branches one after another, so separate launches cost the
+// sum of their durations, where one launch overlaps them. Otherwise the cell
+// list comes first; PME, the longest branch, stays on the context's stream,
+// and the list search with the direct space, and the bonded terms, run on side
+// streams forked after it and joined before anything that reads the forces.
+// Forces are int64 atomics and every energy has its own slot row, so the
+// results do not depend on the overlap.
 // `molecular`: energies with the molecular scaling term; `cellsBuilt`: the
 // step's integrator has built the cell list; `rebuilding`: the list is rebuilt
 // for certain, so its search takes a launch of its own, every row's wave at

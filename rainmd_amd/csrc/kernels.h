@@ -96,7 +96,7 @@ void pmeSetBoxAndInfluence(const PmeDev &p, const BoxF &box, BoxF *dst, const do
 void pmeSetBoxAndInfluenceFrom(const PmeDev &p, const BoxF *box, BoxF *dst, const double *moduli[3], double alpha,
                                hipStream_t s);
 int launchPme(const Dev &d, const PmeDev &p, int energies, hipStream_t s, int *slotsUsed);
-// A small system's direct space, bonded terms and PME forward planes in one
+// A system's direct space, bonded terms and PME forward planes in one
 // launch (where forcesJoin allows), with the energy slots each part used;
 // launchPmeAfterForward then runs the rest of the plane pipeline and returns
 // its slots. With `search` (the one-wave-per-atom list search) a rebuild's

@@ -390,12 +390,15 @@ int launchNonbonded(const Dev &d, float alpha, int rational, int lanes, int ener
 // The joined launch holds the bonded and PME bodies' registers (about 95
 // VGPRs against the direct space's 63 at 64 lanes): a system joins when its
 // direct space fits in one pass at four waves per SIMD of the 256 CUs, as
-// small systems' launch-bound steps do, with the LJ table in LDS, the
-// plane pipeline scanning every atom and at most 64 KB of LDS per workgroup.
+// small and middle systems' do, with the LJ table in LDS, the plane pipeline
+// and at most 64 KB of LDS per workgroup. (12,022 atoms, planes by cells: 97.3
+// us a step apart, 86.3 joined. Past one pass the direct space loses as much
+// to the registers as the overlap gives: 24,022 atoms at 1.2 nm, 149 us a
+// step either way.)
 bool forcesJoin(const Dev &d, const PmeDev &p, int lanes) {
   constexpr long long ONE_PASS = 256LL * 4 * 4 * 64;  // threads
   return (lanes == 16 || lanes == 32 || lanes == 64) && (long long)d.n * lanes <= ONE_PASS && d.typeInList &&
-         p.planes && p.atoms == PME_ATOMS_SCAN && std::max(tableLdsBytes(d), pmePlaneForwardLds(p)) <= 65536;
+         p.planes && p.atoms != PME_ATOMS_BINS && std::max(tableLdsBytes(d), pmePlaneForwardLds(p)) <= 65536;
 }
 
 void launchForcesJoined(const Dev &d, const PmeDev &p, float alpha, int rational, int lanes, int energies,

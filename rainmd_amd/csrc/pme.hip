@@ -830,9 +830,12 @@ bool pmeConfigure(PmeDev &p, int mode, size_t maxLds) {
 
 static int xLineBlocks(const PmeDev &p) { return p.K[1] * ((p.K2h + XLINES - 1) / XLINES); }
 int pmeXLineBlocks(const PmeDev &p) { return xLineBlocks(p); }
-// (A batch member's planes never use the scan list: its LDS is left out.)
+// For a PLANE_THREADS-thread workgroup. (A batch member's planes never use the
+// scan list: its LDS is left out; by cells only the waves' queues are used.)
 size_t pmePlaneForwardLds(const PmeDev &p) {
-  return planeForwardLds(p) - (p.atoms == PME_ATOMS_BINS ? listBytes() : 0);
+  const size_t queues = (size_t)PLANE_THREADS / 64 * QUEUE_ENTRIES * sizeof(PlaneEntry);
+  return planeForwardLds(p) - (p.atoms == PME_ATOMS_SCAN ? 0 : listBytes()) +
+         (p.atoms == PME_ATOMS_CELLS ? queues : 0);
 }
 size_t pmeXLinesLds(const PmeDev &p) { return xLinesLds(p); }
 size_t pmePlaneGatherLds(const PmeDev &p) {
