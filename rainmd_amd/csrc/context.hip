@@ -1192,6 +1192,7 @@ void create(rmd_ctx *c, const System &sys, const rmd_options &o, const Streams *
   }
   d.cellOfAtom = devAlloc<int>(d.nPad, c->held);
   d.cellAtoms = devAlloc<int>(d.nPad, c->held);
+  d.cellArrival = devAlloc<int>(d.nPad, c->held);
   d.cellPos = devAlloc<float4>(d.nPad, c->held);
   d.slotPos = devAlloc<float4>(d.nPad, c->held);
   d.slotType = devAlloc<int>(d.nPad, c->held);

@@ -98,6 +98,7 @@ struct Dev {
   const BoxF *box;  // device-resident geometry (see BoxF)
   // cells (arrays sized for cellCapacity cells)
   int *cellOfAtom, *cellCount, *cellStart, *cellCursor, *cellAtoms;
+  int *cellArrival;  // the atoms by cell as the scatter leaves them, before each cell is put in index order
   float4 *cellPos;  // positions in cell order at the last rebuild, the atom index in .w (int bits; with
                     // typeInList its type above it, as in a list entry)
   int cellCapacity;

@@ -19,7 +19,7 @@
 
 namespace rmd {
 
-constexpr int SORT_CAPACITY = 4096;  // atoms per cell the LDS sort takes
+constexpr int SORT_CAPACITY = 4096;  // atoms per cell the sort takes: its work goes with the square
 
 __global__ void setRebuildKernel(Scalars *sc) {
   sc->rebuild = 1u;
@@ -134,90 +134,46 @@ __global__ void cellsScatterKernel(Dev d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= d.n) return;
   const int slot = atomicAdd(&d.cellCursor[d.cellOfAtom[i]], 1);
-  d.cellAtoms[slot] = i;
+  d.cellArrival[slot] = i;
 }
 
-// The scatter leaves each cell's atoms in arrival order; sorting each cell's
-// run puts them in index order so the list, and every sum over it, is the
-// same on every run. Sorted cells also get their slots written (positions in
-// cell order, with the atom index in .w, for the candidate scan). A workgroup
-// takes CELLS_PER_SORT cells: those of at most SHORT_CELL atoms - every cell
-// of a plan whose cells are a fraction of the list cutoff - are sorted by one
-// thread each, by insertion in that thread's slice of LDS; longer ones then
-// by a bitonic sort over the workgroup, in the same LDS.
-constexpr int SHORT_CELL = 32;
-constexpr int CELLS_PER_SORT = 128;
+// The scatter leaves each cell's atoms in arrival order; putting them in index
+// order makes the list, and every sum over it, the same on every run, and the
+// slots are written with it (positions in cell order, with the atom index in
+// .w, for the candidate scan). One thread per atom counts the atoms of its
+// cell that come before it: the threads of a wave are neighbours in the
+// arrival order, so most of them read the same run at the same time, and the
+// work is spread over the chip however few or crowded the cells are. (A thread
+// per short cell and a workgroup's bitonic sort, cell after cell, for the
+// others took 50 us at 24,022 atoms in cells of 190 or more; this takes 7, and 8
+// at 180,022 atoms.)
+constexpr int RANK_THREADS = 1024;  // few workgroups to start on the steps that keep the list
 
-__global__ void __launch_bounds__(CELLS_PER_SORT) cellsSortKernel(Dev d) {
+__global__ void __launch_bounds__(RANK_THREADS) cellsSortKernel(Dev d) {
   if (!d.sc->rebuild) return;
-  // +1: the threads' slices start in different banks
-  constexpr int SLICE = SHORT_CELL + 1;
-  __shared__ int keys[CELLS_PER_SORT * SLICE > SORT_CAPACITY ? CELLS_PER_SORT * SLICE : SORT_CAPACITY];
-  const int total = d.box->cellTotal, first = blockIdx.x * CELLS_PER_SORT;
-  const int c = first + threadIdx.x;
-  const int begin = c < total ? d.cellStart[c] : 0, len = c < total ? d.cellStart[c + 1] - begin : 0;
-  if (len <= SHORT_CELL) {
-    int *k = keys + threadIdx.x * SLICE;
-    // the cell's atoms loaded together, then sorted in LDS
-    for (int a = 0; a < len; ++a) k[a] = d.cellAtoms[begin + a];
-    for (int a = 1; a < len; ++a) {
-      const int v = k[a];
-      int m = a - 1;
-      while (m >= 0 && k[m] > v) {
-        k[m + 1] = k[m];
-        --m;
-      }
-      k[m + 1] = v;
-    }
-    // positions and types SLOT_BATCH at a time, loaded before any slot is
-    // written (a slot's stores would otherwise wait on its own loads, one
-    // round trip per atom)
-    constexpr int SLOT_BATCH = 4;
-    for (int a = 0; a < len; a += SLOT_BATCH) {
-      float4 p[SLOT_BATCH];
-      int type[SLOT_BATCH];
+  const int k = blockIdx.x * RANK_THREADS + threadIdx.x;
+  if (k >= d.n) return;
+  const int atom = d.cellArrival[k];
+  const float4 p = d.pos[atom];
+  const int type = d.type[atom];
+  const int c = d.cellOfAtom[atom];
+  const int begin = d.cellStart[c], end = d.cellStart[c + 1];
+  int slot = begin;
+  if (end - begin > SORT_CAPACITY) {
+    atomicMax(&d.sc->cellOverflow, 1u);  // the evaluation is refused: any order will do
+    slot = k;
+  } else {
+    int m = begin;
+    for (; m + 8 <= end; m += 8) {
+      int other[8];
 #pragma unroll
-      for (int u = 0; u < SLOT_BATCH; ++u) {
-        const int atom = k[min(a + u, len - 1)];
-        p[u] = d.pos[atom];
-        type[u] = d.type[atom];
-      }
+      for (int u = 0; u < 8; ++u) other[u] = d.cellArrival[m + u];
 #pragma unroll
-      for (int u = 0; u < SLOT_BATCH; ++u)
-        if (a + u < len) writeSlotLoaded(d, begin + a + u, k[a + u], p[u], type[u]);
+      for (int u = 0; u < 8; ++u) slot += other[u] < atom;
     }
+    for (; m < end; ++m) slot += d.cellArrival[m] < atom;
   }
-  if (!__syncthreads_or(len > SHORT_CELL)) return;
-  for (int q = first; q < min(total, first + CELLS_PER_SORT); ++q) {
-    const int b = d.cellStart[q], n = d.cellStart[q + 1] - b;
-    if (n <= SHORT_CELL) continue;
-    if (n > SORT_CAPACITY) {
-      if (threadIdx.x == 0) atomicMax(&d.sc->cellOverflow, 1u);
-      continue;
-    }
-    int size = 1;
-    while (size < n) size <<= 1;
-    for (int k = threadIdx.x; k < size; k += blockDim.x) keys[k] = k < n ? d.cellAtoms[b + k] : 0x7fffffff;
-    __syncthreads();
-    for (int k = 2; k <= size; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int t = threadIdx.x; t < size; t += blockDim.x) {
-          const int partner = t ^ j;
-          if (partner > t) {
-            const bool ascending = (t & k) == 0;
-            const int x = keys[t], y = keys[partner];
-            if ((x > y) == ascending) {
-              keys[t] = y;
-              keys[partner] = x;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    }
-    for (int k = threadIdx.x; k < n; k += blockDim.x) writeSlot(d, b + k, keys[k]);
-    __syncthreads();  // keys is reused for the workgroup's next cell
-  }
+  writeSlotLoaded(d, slot, atom, p, type);
 }
 
 // The whole cell list of a small system in one workgroup: assignment with
@@ -225,8 +181,8 @@ __global__ void __launch_bounds__(CELLS_PER_SORT) cellsSortKernel(Dev d) {
 // wave ballots where there are at most FEW_MAX_CELLS cells (cellsBuildFew),
 // else an LDS scatter and a sort of each cell's run (insertion by one thread
 // per cell, or where a cell is crowded a rank sort: rank = atoms of the same
-// cell with a lower index) - the same lists as the four-kernel path, with no
-// global atomics and three launches fewer on every step. Used when the atoms
+// cell with a lower index) - the same lists as the three-kernel path, with no
+// global atomics and two launches fewer on every step. Used when the atoms
 // and the cells fit the LDS arrays below.
 constexpr int SMALL_THREADS = 1024;
 constexpr int SMALL_MAX_ATOMS = 16384;
@@ -440,8 +396,8 @@ void launchCells(const Dev &d, hipStream_t s) {
     return;
   }
   cellsAssignKernel<<<(d.n + SCAN_THREADS - 1) / SCAN_THREADS, SCAN_THREADS, 0, s>>>(d);
-  cellsScatterKernel<<<(d.n + 255) / 256, 256, 0, s>>>(d);
-  cellsSortKernel<<<(d.cellCapacity + CELLS_PER_SORT - 1) / CELLS_PER_SORT, CELLS_PER_SORT, 0, s>>>(d);
+  cellsScatterKernel<<<(d.n + RANK_THREADS - 1) / RANK_THREADS, RANK_THREADS, 0, s>>>(d);
+  cellsSortKernel<<<(d.n + RANK_THREADS - 1) / RANK_THREADS, RANK_THREADS, 0, s>>>(d);
 }
 
 // The per-cell search runs in the per-atom search's launch (4 waves per
